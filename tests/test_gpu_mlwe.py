@@ -115,6 +115,31 @@ def test_keyswitch_schedules(lib, N, L, K, r, relin, fused, bits):
         lib.vfhe_hip_set_option(b"ks.fused", old)
 
 
+@pytest.mark.parametrize("N,L,K,batch,top", [
+    (8192, 1, 1, 1, False),     # one digit, 8 key blocks
+    (8192, 4, 1, 3, False),     # sums centred on the last digit; 20 key blocks (not a multiple of 8)
+    (8192, 9, 2, 2, True),      # two centrings and a remainder, every residue q - 1
+    (16384, 5, 3, 1, False),    # 6-stage column pass, one digit past a centring
+    (32768, 2, 1, 2, True),
+])
+def test_row_mac_digit_and_tile_shapes(lib, N, L, K, batch, top):
+    """The fused row pass + key inner product over its digit loop, key-block orders and column-pass
+    sizes, against the oracle; `top`: every operand at its largest residue."""
+    s = Setup(N, L, K, 500 + N + L)
+    if top:
+        s.rows = lambda mask: np.stack([np.full(N, (q - 1) if (mask >> i) & 1 else 0, dtype=np.uint64)
+                                        for i, q in enumerate(s.primes)])
+    key = s.key(L, 1)
+    ksk = s.outer([key])
+    ins = [s.ct(1, s.lvl_mask) for _ in range(batch)]
+    outs = [s.pool.sample(1, s.ext_mask) for _ in range(batch)]
+    lib.vfhe_hip_mlwe_keyswitch_batch(_native.voidp_array(outs), _native.voidp_array([c for _, c in ins]), batch, ksk)
+    for (din, _), out in zip(ins, outs):
+        ref = np.zeros((2, L + K, N), dtype=np.uint64)
+        mref = s.octx.ghs_keyswitch(ref, 1, din, 1, s.lvl_mask, [key[0]], s.ext_mask)
+        s.check(s.pool.read_sample(out), ref, mref)
+
+
 def test_multiply_and_batched_rescale(lib):
     """mlwe_multiply (mlwe.c:711-760) and the fused multiply+relinearize+rescale batch."""
     s = Setup(4096, 4, 1, 21)

@@ -70,6 +70,45 @@ template <typename T> __device__ __forceinline__ const VH_GLOBAL T *vh_global(co
 }
 template <typename T> __device__ __forceinline__ VH_GLOBAL T *vh_global(T *p) { return (VH_GLOBAL T *)p; }
 
+// Streaming accesses of the passes: every row is read once and written once per
+// pass, so loads and stores are non-temporal (measured: ~5% on a round trip
+// over 64 x 24 rows of 2^16 against ordinary accesses).
+#ifndef VH_NT_STORE
+#define VH_NT_STORE 1
+#endif
+#ifndef VH_NT_LOAD
+#define VH_NT_LOAD 1
+#endif
+__device__ __forceinline__ void vh_st(VH_GLOBAL uint64_t *p, uint64_t v)
+{
+    if (VH_NT_STORE) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+__device__ __forceinline__ uint64_t vh_ld(const VH_GLOBAL uint64_t *p)
+{
+    if (VH_NT_LOAD) return __builtin_nontemporal_load(p);
+    return *p;
+}
+
+// Two adjacent words as one 16-byte access (rows are 256-byte aligned, p at an even index):
+// an ordinary load, and a streaming store.
+typedef uint64_t vh_u64x2 __attribute__((ext_vector_type(2)));
+typedef double vh_f64x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void vh_ld2(const VH_GLOBAL uint64_t *p, uint64_t &a, uint64_t &b)
+{
+    const vh_u64x2 v = *(const VH_GLOBAL vh_u64x2 *)p;
+    a = v.x;
+    b = v.y;
+}
+__device__ __forceinline__ void vh_st2(VH_GLOBAL uint64_t *p, uint64_t a, uint64_t b)
+{
+    vh_u64x2 v;
+    v.x = a;
+    v.y = b;
+    if (VH_NT_STORE) __builtin_nontemporal_store(v, (VH_GLOBAL vh_u64x2 *)p);
+    else *(VH_GLOBAL vh_u64x2 *)p = v;
+}
+
 #define VH_MAGIC 6755399441055744.0   /* 1.5 * 2^52 */
 #define VH_TWO52 4503599627370496.0   /* 2^52 */
 

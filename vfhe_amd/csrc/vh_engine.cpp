@@ -2303,7 +2303,7 @@ struct vh_gsrc {
     RNS_MLWE *keys;
 };
 
-// The fused ModUp row pass + key inner product (k_ntt16_row_mac) runs when every limb of
+// The fused ModUp row pass + key inner product (k_row_mac) runs when every limb of
 // `mask` is on the FP64 path, the ring is not split, N = 2^13..2^16 and the output has at
 // most two components.
 static bool fused_mac_ok(incNTT t, uint64_t mask, uint64_t comps)
@@ -2483,8 +2483,8 @@ static void gadget_batch(const std::vector<RNS_MLWE> &outs, const std::vector<st
                 {
                     vh_prof_scope ps_(VH_PROF_KSMAC);
                     if (fused_mac)
-                        VH_LAUNCH(vh_launch_ntt16_row_mac(S(), vh_stage_vec(chunk), cnt, (unsigned)maxnext, P->d_limbs,
-                                                         d_kptr, logn, (int)Cc));
+                        VH_LAUNCH(vh_launch_row_mac(S(), vh_stage_vec(chunk), cnt, (unsigned)maxnext, P->d_limbs,
+                                                   d_kptr, logn, (int)Cc));
                     else
                         VH_LAUNCH(vh_launch_keyswitch_mac(S(), vh_stage_vec(chunk), cnt, (unsigned)maxnext, P->d_limbs,
                                                          d_kptr, N, fp_mac ? 1 : 0));

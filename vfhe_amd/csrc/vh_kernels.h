@@ -186,8 +186,8 @@ hipError_t vh_launch_permute(hipStream_t st, const vh_item *items, unsigned nite
 // Forward row pass (last 8 stages) of every digit fused with the inner product
 // out_c = -sum_d digit_d * key[d][c]; modup holds the column-pass output.
 // FP64 path, 13 <= logn <= 16, comps 1 or 2.
-hipError_t vh_launch_ntt16_row_mac(hipStream_t st, const vh_mac_job *jobs, unsigned njobs, unsigned next,
-                                   const vh_limb *limbs, const uint64_t *const *kptr, int logn, int comps);
+hipError_t vh_launch_row_mac(hipStream_t st, const vh_mac_job *jobs, unsigned njobs, unsigned next,
+                             const vh_limb *limbs, const uint64_t *const *kptr, int logn, int comps);
 // Forward row stages of it.src and it.src2 (column-pass outputs), their pointwise
 // product and the inverse row stages, into it.dst (the inverse column pass input).
 // Pipelined form of the same step (persistent workgroups, cus x its occupancy, or one tile per

@@ -147,26 +147,6 @@ k_ntt_pass(const vh_item *__restrict__ items, const vh_limb *__restrict__ limbs,
 // private to it, so their exchanges only need the wave's own LDS operations to
 // stay in program order (vh_wave_sync).
 
-// Streaming accesses of the passes: every row is read once and written once per
-// pass, so loads and stores are non-temporal (measured: ~5% on a round trip
-// over 64 x 24 rows of 2^16 against ordinary accesses).
-#ifndef VH_NT_STORE
-#define VH_NT_STORE 1
-#endif
-#ifndef VH_NT_LOAD
-#define VH_NT_LOAD 1
-#endif
-__device__ __forceinline__ void vh_st(VH_GLOBAL uint64_t *p, uint64_t v)
-{
-    if (VH_NT_STORE) __builtin_nontemporal_store(v, p);
-    else *p = v;
-}
-__device__ __forceinline__ uint64_t vh_ld(const VH_GLOBAL uint64_t *p)
-{
-    if (VH_NT_LOAD) return __builtin_nontemporal_load(p);
-    return *p;
-}
-
 template <int R, bool COL> constexpr int vh_ntt16_lds()
 {
     return COL ? (1 << R) * (256 / ((1 << R) / 16) + 1) : (256 / ((1 << R) / 16)) * ((1 << R) + (1 << R) / 16);
@@ -575,216 +555,6 @@ k_ntt16p(const vh_item *__restrict__ items, const vh_limb *__restrict__ limbs, i
             }
         }
     }
-}
-
-// ---------------------------------------------------------------------------
-// Key-switch inner product fused into the forward row pass (FP64 path,
-// N = 2^13..2^16, at most 2 output components).  The column pass has left the
-// lifted digit rows, transformed over their first logn-8 stages, in jb.modup;
-// this kernel finishes the last 8 stages of every digit for one 4096-element
-// block and accumulates   out_c = - sum_d NTT(digit_d) * key[d][c]   (the
-// mul_subto of gadget.c:22-37) in registers, so the transformed digits never
-// return to memory.  Grid: x = ciphertext, y = 4096-element block, z = extended
-// limb; a key block is (y, z).  Consecutive workgroups are dealt round-robin
-// over the 8 XCDs, so with `xcd` set the workgroup index is remapped to put all
-// ciphertexts of one key block on one XCD, one after another: each XCD's L2 then
-// fetches a key block once instead of every XCD fetching it.
-// ---------------------------------------------------------------------------
-template <int C>
-__global__ void __launch_bounds__(256)
-k_ntt16_row_mac(const vh_mac_job *__restrict__ jobs, const vh_limb *__restrict__ limbs,
-                const uint64_t *const *__restrict__ kptr, int logn, int xcd)
-{
-    constexpr int R = 8, S = 256, TPS = 16, G = 16;
-    __shared__ double lds[vh_ntt16_lds<R, false>()];
-    unsigned bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
-    if (xcd) {   // bijective when gridDim.y * gridDim.z is a multiple of 8 (checked at launch)
-        const unsigned lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-        const unsigned slot = lin >> 3, kb = (slot / gridDim.x) * 8 + (lin & 7);
-        bx = slot % gridDim.x;
-        by = kb % gridDim.y;
-        bz = kb / gridDim.y;
-    }
-    const vh_mac_job &jb = jobs[bx];
-    const int ti = (int)bz, D = jb.digits;
-    if (ti >= jb.next) return;   // jobs of a batch may have fewer extended limbs (whole block)
-    const int limb = jb.limb[ti];
-    const vh_limb &L = limbs[limb];
-    const double q = L.qd, qinv = L.qinv;
-    const size_t n = (size_t)1 << logn;
-    const int s0 = logn - R;
-    const int tid = threadIdx.x, g = tid / TPS, t = tid % TPS;
-    const size_t sub = (size_t)by * G + g;
-    const VH_GLOBAL double *tw = vh_global(reinterpret_cast<const double *>(L.tw_fwd));
-    auto lidx = [&](int k) -> int { return g * (S + S / 16) + k + (k >> 4); };
-    // Twiddles do not depend on the digit: they are staged in LDS once, so the digit
-    // loop issues no twiddle load behind the next digit's prefetch.  rowt[g]: the 15
-    // stride-stage twiddles of row g; head: tw[0..255]; rowb[g]: row g's factors of
-    // stages 4..7 (contiguous-stage twiddle = head entry * factor, as in k_ntt16p).
-    __shared__ double2 head[256], rowt[G][15], rowb[G][4];
-    {
-        const int tid0 = threadIdx.x;
-        head[tid0] = make_double2(tw[2 * tid0], tw[2 * tid0 + 1]);
-        if (tid0 < G * 15) {
-            const int r = tid0 / 15, e = tid0 % 15;           // e = 2^sp - 1 + local
-            const int sp = 31 - __builtin_clz(e + 1), local = e + 1 - (1 << sp);
-            const size_t i = ((size_t)1 << (s0 + sp)) + (((size_t)by * G + r) << sp) + local;
-            rowt[r][e] = make_double2(tw[2 * i], tw[2 * i + 1]);
-        }
-        if (tid0 < G * 4) {
-            const int r = tid0 / 4, k = tid0 % 4;
-            const VH_GLOBAL double *rf = vh_global(reinterpret_cast<const double *>(L.rowf_fwd));
-            const size_t i = ((size_t)by * G + r) * 8 + 4 + k;
-            rowb[r][k] = make_double2(rf[2 * i], rf[2 * i + 1]);
-        }
-        __syncthreads();
-    }
-    auto twid = [&](int sp, size_t local) -> double2 {
-        if (sp < 4) return rowt[g][(1 << sp) - 1 + (int)local];
-        const double2 h = head[(1 << sp) + (int)local], b = rowb[g][sp - 4];
-        const double w = vh_center(vh_mulmod_tw(h.x, b.x, b.y, q), q, qinv);
-        return make_double2(w, w * qinv);
-    };
-    auto digit_row = [&](int d) -> const VH_GLOBAL uint64_t * {
-        return vh_global(jb.modup + ((size_t)d * jb.next + ti) * n + sub * S);
-    };
-    // After the last stage a thread owns the contiguous elements x0 .. x0+15 of its
-    // row: key rows are read and outputs written as 16 consecutive words per lane.
-    const size_t x0 = sub * S + 16 * t;
-
-    double acc[C][16];
-#pragma unroll
-    for (int c = 0; c < C; c++)
-#pragma unroll
-        for (int m = 0; m < 16; m++) acc[c][m] = 0.0;
-
-    // One output component: the next digit is prefetched and the key words load with it,
-    // so both land during the butterflies.  Two components: the 64 accumulator registers
-    // leave room for neither (the prefetching form needs 238 VGPRs, two waves per SIMD);
-    // the digit and then each component's key words load when needed, at 162 VGPRs and
-    // three waves per SIMD, whose extra wave hides those loads (3% faster, measured).
-    constexpr bool PREF = C == 1, KEARLY = C == 1;
-    uint64_t raw[16];
-    if (D > 0 && PREF) {
-        const VH_GLOBAL uint64_t *in = digit_row(0);
-#pragma unroll
-        for (int m = 0; m < 16; m++) raw[m] = vh_ld(in + t + TPS * m);
-    }
-    for (int d = 0; d < D; d++) {
-        double v[16];
-        if (!PREF) {
-            const VH_GLOBAL uint64_t *in = digit_row(d);
-#pragma unroll
-            for (int m = 0; m < 16; m++) raw[m] = vh_ld(in + t + TPS * m);
-        }
-#pragma unroll
-        for (int m = 0; m < 16; m++) v[m] = __longlong_as_double((long long)raw[m]);
-        if (PREF && d + 1 < D) {   // next digit's loads overlap this digit's butterflies
-            const VH_GLOBAL uint64_t *in = digit_row(d + 1);
-#pragma unroll
-            for (int m = 0; m < 16; m++) raw[m] = vh_ld(in + t + TPS * m);
-        }
-        const uint64_t *const *kp = kptr + jb.kptr_off + ((size_t)ti * D + d) * C;
-        uint64_t kw[C][16];
-        if (KEARLY) {
-#pragma unroll
-            for (int c = 0; c < C; c++) {
-                const VH_GLOBAL uint64_t *kr = vh_global(kp[c]) + x0;
-#pragma unroll
-                for (int m = 0; m < 16; m++) kw[c][m] = kr[m];
-            }
-        }
-        // stages s' = 0..3, stride ownership
-#pragma unroll
-        for (int sp = 0; sp < 4; sp++) {
-            const int hm = 8 >> sp;
-#pragma unroll
-            for (int m = 0; m < 16; m++) {
-                if (m & hm) continue;
-                const double2 w = twid(sp, (size_t)(m >> (4 - sp)));
-                const double x = vh_mulmod_tw(v[m + hm], w.x, w.y, q);
-                const double u = v[m];
-                v[m] = u + x;
-                v[m + hm] = u - x;
-            }
-        }
-        vh_wave_sync();  // every read of the previous digit's exchange is done
-#pragma unroll
-        for (int m = 0; m < 16; m++) lds[lidx(t + TPS * m)] = vh_center(v[m], q, qinv);
-        vh_wave_sync();
-#pragma unroll
-        for (int m = 0; m < 16; m++) v[m] = lds[lidx(16 * t + m)];
-        // stages s' = 4..7, contiguous ownership
-#pragma unroll
-        for (int sp = 4; sp < R; sp++) {
-            const int hm = 1 << (R - sp - 1);
-#pragma unroll
-            for (int m = 0; m < 16; m++) {
-                if (m & hm) continue;
-                const double2 w = twid(sp, (size_t)((16 * t + m) >> (R - sp)));
-                const double x = vh_mulmod_tw(v[m + hm], w.x, w.y, q);
-                const double u = v[m];
-                v[m] = u + x;
-                v[m + hm] = u - x;
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < C; c++) {
-            if (!KEARLY) {
-                const VH_GLOBAL uint64_t *kr = vh_global(kp[c]) + x0;
-#pragma unroll
-                for (int m = 0; m < 16; m++) kw[c][m] = kr[m];
-            }
-#pragma unroll
-            for (int h = 0; h < 8; h++) {
-#pragma unroll
-                for (int e = 0; e < 2; e++) {
-                    const int m = 2 * h + e;
-                    const double a = vh_center(v[m], q, qinv);          // |a| <= q/2 + 1
-                    const double k = vh_u2d(kw[c][m]);
-                    const double hi = a * k;
-                    const double lo = __fma_rn(a, k, -hi);
-                    const double qt = __fma_rn(a, k * qinv, VH_MAGIC) - VH_MAGIC;
-                    const double r = __fma_rn(-qt, q, hi) + lo;   // |r| <= q + 2^47
-                    // centred every 4th digit: |acc| <= q/2 + 4 (q + 2^47) < 2^53 stays exact
-                    acc[c][m] = (d & 3) == 3 ? vh_center(acc[c][m] + r, q, qinv) : acc[c][m] + r;
-                }
-            }
-        }
-    }
-    const bool fold = (jb.pass_mask >> limb) & 1;
-#pragma unroll
-    for (int c = 0; c < C; c++) {
-        VH_GLOBAL uint64_t *out = vh_global(jb.out[c] + (size_t)limb * n + x0);
-        if (fold && jb.pass[c]) {
-            // |acc| <= q/2 + 4 (q + 2^47) and |P d| <= 3q/4: the sum stays below 2^53.  A lane
-            // reads 16 consecutive words (ordinary loads, merged into wide ones, like the key words).
-            const VH_GLOBAL uint64_t *ps = vh_global(jb.pass[c] + (size_t)limb * n + x0);
-            const double2 pm = jb.pmod[limb];
-            uint64_t pw[16];
-#pragma unroll
-            for (int m = 0; m < 16; m++) pw[m] = ps[m];
-#pragma unroll
-            for (int m = 0; m < 16; m++) {
-                const double y = (jb.add ? acc[c][m] : -acc[c][m]) + vh_mulmod_tw(vh_u2d(pw[m]), pm.x, pm.y, q);
-                vh_st(out + m, vh_d2u(vh_canon(y, q, qinv)));
-            }
-        } else {
-#pragma unroll
-            for (int m = 0; m < 16; m++) vh_st(out + m, vh_d2u(vh_canon(jb.add ? acc[c][m] : -acc[c][m], q, qinv)));
-        }
-    }
-}
-
-hipError_t vh_launch_ntt16_row_mac(hipStream_t st, const vh_mac_job *jobs, unsigned njobs, unsigned next,
-                                   const vh_limb *limbs, const uint64_t *const *kptr, int logn, int comps)
-{
-    if (logn < 13 || logn > 16 || comps < 1 || comps > 2) return hipErrorInvalidValue;
-    const dim3 grid(njobs, 1u << (logn - 12), next);
-    const int xcd = (grid.y * grid.z) % 8 == 0;
-    if (comps == 1) VH_KL(k_ntt16_row_mac<1>, grid, dim3(256), 0, st, jobs, limbs, kptr, logn, xcd);
-    else VH_KL(k_ntt16_row_mac<2>, grid, dim3(256), 0, st, jobs, limbs, kptr, logn, xcd);
-    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
