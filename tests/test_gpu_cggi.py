@@ -17,7 +17,7 @@ import random
 import numpy as np
 import pytest
 
-from vfhe_amd import _native, arith
+from vfhe_amd import _native, arith, params, runtime as rt
 from vfhe_amd.arith import Ring
 from vfhe_amd.cggi import BootstrapKey, Bootstrapper, LweBatch, LweKey, extract, lwe_key_of, pack_lut, rotation_amounts
 from vfhe_amd.cggi import _LweStruct as LweStruct
@@ -278,3 +278,45 @@ def test_bootstrap_batch_shape_n630_N1024():
     phases = out.phases(lwe_key_of(out_key, in_ring))
     got = [mod_switch(ph, q, 1 << MSG_PREC) for ph in phases]
     assert got == msgs
+
+
+@pytest.mark.parametrize("rank,nj,count,bits", [
+    (1, 2, 1, 50), (1, 2, 259, 50), (1, 1, 3, 50), (1, 1, 257, 50), (1, 3, 5, 50), (1, 3, 258, 50),
+    (0, 1, 2, 50), (0, 2, 3, 50), (0, 2, 257, 50), (0, 3, 2, 50), (1, 2, 4, 30),
+])
+def test_fused_blind_rotation_shapes(rank, nj, count, bits):
+    """Every form of the one-launch blind rotation (one accumulator per workgroup with one or two
+    groups of waves, two accumulators per workgroup with the last slot empty) against the launch
+    sequence per key index, bit for bit: uniform keys, exponents at 0, 1, N - 1, N, 2N - 1."""
+    N, n = 1024, 7
+    lib = _native.load()
+    primes = params.gen_primes(N, [bits] * (nj + 1))
+    pool = rt.Pool(N, primes)
+    rng = np.random.default_rng(7000 + 100 * nj + 10 * rank + count)
+    full, level = (1 << (nj + 1)) - 1, (1 << nj) - 1
+
+    def sample(mask):
+        return pool.sample(rank, mask, np.stack([rt.random_rows(rng, primes, N, mask) for _ in range(rank + 1)]))
+
+    keys = [_native.voidp_array([sample(full) for _ in range((rank + 1) * nj)]) for _ in range(n)]
+    table = _native.voidp_array(keys)
+    tv = sample(level)
+    steps = rng.integers(0, 2 * N, (count, n), dtype=np.uint64)
+    steps[0, :5] = [0, 1, N - 1, N, 2 * N - 1]
+    rots = rng.integers(0, 2 * N, count, dtype=np.uint64)
+    saved = lib.vfhe_hip_get_option(b"br.fused")
+    got = {}
+    try:
+        for fused in (1, 0):
+            assert lib.vfhe_hip_set_option(b"br.fused", fused) == 0
+            n0 = lib.vfhe_hip_get_option(b"stat.br_fused_launches")
+            acc = [pool.sample(rank, level) for _ in range(count)]
+            print(f"[cggi] rank={rank} limbs={nj} count={count} fused={fused}", flush=True)
+            lib.vfhe_hip_blind_rotate_tv_batch(_native.voidp_array(acc), count, tv, rots.ctypes.data_as(_native.U64P),
+                                               table, n, steps.ctypes.data_as(_native.U64P), nj, 1)
+            assert (lib.vfhe_hip_get_option(b"stat.br_fused_launches") - n0) == fused
+            got[fused] = [pool.read_sample(c)[:, :nj] for c in acc]
+    finally:
+        lib.vfhe_hip_set_option(b"br.fused", saved)
+    for k in range(count):
+        assert np.array_equal(got[1][k], got[0][k]), k

@@ -3291,6 +3291,8 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
             bp.hdiv[w] = (double)((p / 2) % qe);
             bp.inv[w] = centred(iv, qe);
             bp.invq[w] = bp.inv[w] / (double)qe;
+            bp.ninv_inv[w] = centred(mulmod_h(t->ntt[E[w]]->h.ninv, iv, qe), qe);
+            bp.ninv_invq[w] = bp.ninv_inv[w] / (double)qe;
         }
         std::vector<uint64_t *> accp(count * Cc * J.size());
         for (uint64_t k = 0; k < count; k++) {
@@ -3346,7 +3348,8 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
         }
         {
             vh_prof_scope ps_(VH_PROF_KSMAC);
-            VH_LAUNCH(vh_launch_blind_rotate(S(), bp, P->d_limbs, d_acc, d_bk, d_am, (unsigned)count, d_tv, d_rot));
+            VH_LAUNCH(vh_launch_blind_rotate(S(), bp, P->d_limbs, d_acc, d_bk, d_am, (unsigned)count,
+                                             (unsigned)C.cus, d_tv, d_rot));
         }
         g_br_fused_launches++;
         if (!held.empty()) {

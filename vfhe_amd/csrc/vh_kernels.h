@@ -92,22 +92,24 @@ struct vh_mac_job {
 // Whole FP64 transforms of N = 2^9 .. 2^12 (reads it.src, writes it.dst), registers radix-16.
 hipError_t vh_launch_ntt_small(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, int dir,
                                int logn);
-// Fused CGGI blind rotation (N = 1024, FP64 limbs, one special prime): workgroup k steps
-// accumulator k through every key index with its rows resident in LDS; wave w works modulo
-// extended limb E[w].
+// Fused CGGI blind rotation (N = 1024, FP64 limbs, one special prime): accumulator k steps
+// through every key index with its rows in its workgroup's registers and LDS; waves 2w and
+// 2w + 1 of an accumulator work modulo extended limb E[w].
 #define VH_BR_MAXE 4
 #define VH_BR_MAXJ 3
 struct vh_br_params {
     int C;                      // components (rank + 1), 1 or 2
     int nJ;                     // level limbs (digits per component)
-    int next;                   // extended limbs = waves per workgroup (nJ + 1)
-    int sp;                     // wave of the special limb
+    int next;                   // extended limbs (nJ + 1)
+    int sp;                     // index in E of the special limb
     int E[VH_BR_MAXE];          // extended limbs, ascending
     int J[VH_BR_MAXJ];          // level limbs, ascending
-    int jw[VH_BR_MAXE];         // wave -> index in J (-1: the special limb)
+    int jw[VH_BR_MAXE];         // index in E -> index in J (-1: the special limb)
     double hdiv[VH_BR_MAXE];    // floor(p/2) mod q_E[w]
     double inv[VH_BR_MAXE];     // p^-1 mod q_E[w], centred
     double invq[VH_BR_MAXE];    // RN(inv / q_E[w])
+    double ninv_inv[VH_BR_MAXE];    // N^-1 p^-1 mod q_E[w], centred
+    double ninv_invq[VH_BR_MAXE];   // RN(ninv_inv / q_E[w])
     double hp;                  // floor(p/2)
     uint64_t n;                 // key indices
 };
@@ -116,7 +118,7 @@ struct vh_br_params {
 // component c, limb E[w] (NTT form); amounts[k * n + i] < 2N.  tvp (optional): the C nJ rows of a
 // test vector; accumulator k then starts as X^rot[k] * tv instead of from its own rows.
 hipError_t vh_launch_blind_rotate(hipStream_t st, const vh_br_params &P, const vh_limb *limbs, uint64_t *const *accp,
-                                  const uint64_t *const *bkp, const uint64_t *amounts, unsigned count,
+                                  const uint64_t *const *bkp, const uint64_t *amounts, unsigned count, unsigned cus,
                                   const uint64_t *const *tvp = nullptr, const uint64_t *rot = nullptr);
 // CGGI over the 32-bit torus (vh_torus.hip).  consts: 576 double2 -- [0, 512) pass 1's
 // twiddles with the lane's twist factor, zeta^r w^(r k) at k 64 + r (r < 64, k < 8),

@@ -1603,153 +1603,6 @@ k_ntt_small(const vh_item *__restrict__ items, unsigned nitems, const vh_limb *_
 }
 
 // ---------------------------------------------------------------------------
-// CGGI16 blind rotation of a batch, every key index in one launch (cggi16.py:70-90 with
-// mgsw.c:51-71 per index).  N = 1024, FP64 limbs, one special prime.  Workgroup k holds
-// accumulator k's level rows in LDS (coefficient form) for the whole loop; wave w works
-// modulo extended limb E[w].  Per key index i with a = amounts[k n + i] != 0:
-//   digit d = (component c, level limb J[jj]):  (X^a - 1) acc_c  at limb J[jj], canonical,
-//     read from LDS straight into the forward transform's registers (the reference's
-//     mlwe_RNSc_mul_by_xai, subtraction and gadget lift; the lift is the identity on
-//     values below q_J[jj] < 2^50, which the FP64 transform accepts for any E[w]);
-//   out_c' += NTT_E[w](digit) * bk[i][d] component c' (FP64 products, centred every 4th
-//     digit), the 16 key words per lane contiguous;
-//   then per c': inverse transform, the special wave publishes t = (x + floor(p/2)) mod p
-//     and every level wave adds (x + floor(p/2) - t) p^-1 mod q to its accumulator row
-//     (round division by p, then the CMUX's  acc + ExtProd(X^a acc - acc)).
-// A zero exponent leaves the accumulator as it is (the reference skips that index).
-// Every wave takes part in every barrier; the exponent is uniform over the workgroup.
-// ---------------------------------------------------------------------------
-template <int C, int NJ>
-__global__ void __launch_bounds__(256, 2)
-k_blind_rotate(const vh_br_params P, const vh_limb *__restrict__ limbs, uint64_t *const *__restrict__ accp,
-               const uint64_t *const *__restrict__ bkp, const uint64_t *__restrict__ amounts,
-               const uint64_t *const *__restrict__ tvp, const uint64_t *__restrict__ rot)
-{
-    using R = vh_reg_ntt<10>;
-    constexpr int N = 1024, PAD = N + N / 16, nJ = NJ, next = NJ + 1, nd = C * NJ;
-    // C NJ rows of the accumulator, one exchange buffer per wave, the special limb's t:
-    // 65.5 KiB for C = 2, NJ = 2 (two workgroups per CU)
-    __shared__ double dyn[C * NJ * N + next * PAD + N];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const unsigned k = blockIdx.x;
-    double *accd = dyn;                           // [C][nJ][N]
-    double *scratch = accd + C * nJ * N + w * PAD; // this wave's exchange buffer
-    double *spd = dyn + C * nJ * N + next * PAD;   // [N]: the special limb's t of one component
-    // the accumulator's rows (every wave helps): its own, or X^rot[k] * tv (the initial
-    // rotation of the test vector, mlwe_RNSc_mul_by_xai: coefficient u = (x - a) mod 2N
-    // of tv, negated when u >= N)
-    for (int r = 0; r < C * nJ; r++) {
-        if (tvp) {
-            const VH_GLOBAL uint64_t *src = vh_global(tvp[r]);
-            const uint32_t a = (uint32_t)(rot[k] & (2 * N - 1));
-            const double qr = limbs[P.J[r % nJ]].qd;
-            for (int x = threadIdx.x; x < N; x += blockDim.x) {
-                const uint32_t u = (uint32_t)(x + 2 * N - a) & (2 * N - 1);
-                const double sv = vh_u2d(src[u & (N - 1)]);
-                accd[r * N + x] = (u < N || sv == 0.0) ? sv : qr - sv;
-            }
-        } else {
-            const VH_GLOBAL uint64_t *src = vh_global(accp[(size_t)k * C * nJ + r]);
-            for (int x = threadIdx.x; x < N; x += blockDim.x) accd[r * N + x] = vh_u2d(src[x]);
-        }
-    }
-    __syncthreads();
-    const vh_limb &L = limbs[P.E[w]];
-    const double q = L.qd, qinv = L.qinv;
-    const VH_GLOBAL double *twf = vh_global(reinterpret_cast<const double *>(L.tw_fwd));
-    const VH_GLOBAL double *twi = vh_global(reinterpret_cast<const double *>(L.tw_inv));
-    const VH_GLOBAL uint64_t *am = vh_global(amounts + (size_t)k * P.n);
-    for (uint64_t i = 0; i < P.n; i++) {
-        const uint32_t a = (uint32_t)(am[i] & (2 * N - 1));
-        if (a == 0) continue;
-        double out[C][16];
-#pragma unroll
-        for (int c = 0; c < C; c++)
-#pragma unroll
-            for (int m = 0; m < 16; m++) out[c][m] = 0.0;
-        for (int d = 0; d < nd; d++) {
-            const int c = d / nJ, jj = d - c * nJ;
-            const double qj = limbs[P.J[jj]].qd;
-            const double *row = accd + (c * nJ + jj) * N;
-            double v[16];
-#pragma unroll
-            for (int m = 0; m < 16; m++) {
-                const int x = R::jA(lane, m);
-                const uint32_t u = (uint32_t)(x + 2 * N - a) & (2 * N - 1);
-                const double s = row[u & (N - 1)];
-                double r = (u < N ? s : -s) - row[x];     // in (-2 q_j, q_j)
-                r = r < 0.0 ? r + qj : r;
-                v[m] = r < 0.0 ? r + qj : r;
-            }
-            R::template fwd<true>(v, scratch, lane, twf, q, qinv);
-            const uint64_t *const *kp = bkp + ((i * nd + d) * C) * next + w;
-#pragma unroll
-            for (int c2 = 0; c2 < C; c2++) {
-                const VH_GLOBAL uint64_t *kr = vh_global(kp[(size_t)c2 * next]) + 16 * lane;
-                uint64_t kw[16];
-#pragma unroll
-                for (int m = 0; m < 16; m++) kw[m] = kr[m];
-#pragma unroll
-                for (int m = 0; m < 16; m++) {
-                    const double x = vh_center(v[m], q, qinv);
-                    const double kk = vh_u2d(kw[m]);
-                    const double hi = x * kk;
-                    const double lo = __fma_rn(x, kk, -hi);
-                    const double qt = __fma_rn(x, kk * qinv, VH_MAGIC) - VH_MAGIC;
-                    const double r = __fma_rn(-qt, q, hi) + lo;   // |r| <= q + 2^47
-                    out[c2][m] = (d & 3) == 3 ? vh_center(out[c2][m] + r, q, qinv) : out[c2][m] + r;
-                }
-            }
-        }
-        __syncthreads();   // every wave has read the accumulator rows of this index
-#pragma unroll
-        for (int c2 = 0; c2 < C; c2++) {
-            double v[16];
-#pragma unroll
-            for (int m = 0; m < 16; m++) v[m] = vh_center(out[c2][m], q, qinv);
-            R::template inv<true>(v, scratch, lane, twi, q, qinv);
-#pragma unroll
-            for (int m = 0; m < 16; m++) v[m] = vh_canon(vh_mulmod_tw(v[m], L.ninv_d, L.ninv_q, q), q, qinv);
-            if (w == P.sp) {
-#pragma unroll
-                for (int m = 0; m < 16; m++) spd[R::jA(lane, m)] = vh_canon(v[m] + P.hp, q, qinv);
-            }
-            __syncthreads();
-            if (w != P.sp) {
-                double *row = accd + (c2 * nJ + P.jw[w]) * N;
-                const double h = P.hdiv[w], iv = P.inv[w], ivq = P.invq[w];
-#pragma unroll
-                for (int m = 0; m < 16; m++) {
-                    const int x = R::jA(lane, m);
-                    const double y = vh_mulmod_tw(v[m] + h - spd[x], iv, ivq, q);
-                    row[x] = vh_canon(row[x] + y, q, qinv);
-                }
-            }
-            __syncthreads();
-        }
-    }
-    for (int r = 0; r < C * nJ; r++) {
-        VH_GLOBAL uint64_t *dst = vh_global(accp[(size_t)k * C * nJ + r]);
-        for (int x = threadIdx.x; x < N; x += blockDim.x) dst[x] = vh_d2u(accd[r * N + x]);
-    }
-}
-
-hipError_t vh_launch_blind_rotate(hipStream_t st, const vh_br_params &P, const vh_limb *limbs, uint64_t *const *accp,
-                                  const uint64_t *const *bkp, const uint64_t *amounts, unsigned count,
-                                  const uint64_t *const *tvp, const uint64_t *rot)
-{
-    if (P.C < 1 || P.C > 2 || P.nJ < 1 || P.nJ > VH_BR_MAXJ || P.next != P.nJ + 1 || P.next > VH_BR_MAXE ||
-        P.sp < 0 || P.sp >= P.next || count == 0 || (tvp && !rot))
-        return hipErrorInvalidValue;
-    const dim3 grid(count), block(64 * P.next);
-#define VH_BR(CC, JJ)                                                                                      \
-    if (P.C == CC && P.nJ == JJ) VH_KL((k_blind_rotate<CC, JJ>), grid, block, 0, st, P, limbs, accp, bkp, amounts, tvp, rot);
-    VH_BR(1, 1) VH_BR(1, 2) VH_BR(1, 3) VH_BR(2, 1) VH_BR(2, 2) VH_BR(2, 3)
-#undef VH_BR
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
 // Batched sample extraction: one thread per output word (grid-stride).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_extract_lwe(const uint64_t *const *__restrict__ src,
