@@ -4643,7 +4643,7 @@ extern "C" int vfhe_hip_torus_bootstrap(vfhe_torus_batch *out, vfhe_torus_batch 
     A.offset = (uint32_t)((1ull << 32) / (4 * torus_base));
     A.dec_off = dec_off;
     vh_prof_scope ps_(VH_PROF_OTHER);
-    VH_LAUNCH(vh_launch_torus_blind_rotate(S(), A, in->count));
+    VH_LAUNCH(vh_launch_torus_blind_rotate(S(), A, in->count, (unsigned)C.cus));
     return 0;
 }
 

@@ -137,7 +137,7 @@ struct vt_br_args {
 };
 hipError_t vh_launch_torus_fft(hipStream_t st, const uint32_t *in, double2 *out, const double2 *consts, uint64_t count,
                                int natural);
-hipError_t vh_launch_torus_blind_rotate(hipStream_t st, const vt_br_args &A, uint64_t count);
+hipError_t vh_launch_torus_blind_rotate(hipStream_t st, const vt_br_args &A, uint64_t count, unsigned cus);
 // Batched sample extraction (mlwe_extract_LWE, mlwe.c:40-66, at coefficient idx): src[(k na + j)
 // (r + 1) + c] = row of limb j of component c of sample k (coefficient form), qs[j] its prime;
 // out[(k na + j) (r N + 1) + e] = the extracted sample's mask words (e < r N) and body (e = r N).

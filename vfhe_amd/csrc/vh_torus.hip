@@ -121,11 +121,48 @@ __device__ __forceinline__ void vt_fill_tw(double2 *t1, double2 *t2, const doubl
     }
 }
 
+// Pass 2's twiddles w^(8 a s) of a = lane mod 8: read from the LDS table, or kept in registers.
+struct vt_t2_lds {
+    const double2 *t;
+    __device__ __forceinline__ double2 operator()(int s, int a) const { return t[(s - 1) * 8 + a]; }
+};
+struct vt_t2_reg {
+    double2 t[8];
+    __device__ __forceinline__ double2 operator()(int s, int) const { return t[s]; }
+};
+
+// One exchange of a lane's eight complex values through LDS: written at w + ws s, read at
+// r + rs s.  SEQ: the real parts, then the imaginary parts, through one array (a wave's LDS
+// operations complete in order), so the second write overlaps the first read.
+template <bool SEQ>
+__device__ __forceinline__ void vt_exchange(double *re, double *im, double *xr, double *xi, int w, int ws, int r, int rs)
+{
+    vh_wave_sync();
+#pragma unroll
+    for (int s = 0; s < 8; s++) xr[w + ws * s] = re[s];
+    if (!SEQ) {
+#pragma unroll
+        for (int s = 0; s < 8; s++) xi[w + ws * s] = im[s];
+    }
+    vh_wave_sync();
+#pragma unroll
+    for (int s = 0; s < 8; s++) re[s] = xr[r + rs * s];
+    if (SEQ) {
+        vh_wave_sync();
+#pragma unroll
+        for (int s = 0; s < 8; s++) xr[w + ws * s] = im[s];
+        vh_wave_sync();
+    }
+#pragma unroll
+    for (int s = 0; s < 8; s++) im[s] = (SEQ ? xr : xi)[r + rs * s];
+}
+
 // Forward transform: layout A in, layout C out.
 // Pass 1's twiddles zeta^r w^(r k) are formed by powers of the lane's w^r from zeta^r
 // (z = {zeta^r, w^r}): seven products instead of eight LDS reads of 16 bytes.
+template <bool SEQ = false, typename T2>
 __device__ __forceinline__ void vt_fwd(double *re, double *im, double *xr, double *xi, const double2 (&z)[2],
-                                       const double2 *t2, int lane)
+                                       const T2 &t2, int lane)
 {
     const int hi = lane >> 3, lo = lane & 7;
     vt_dft8<-1>(re, im);
@@ -137,75 +174,32 @@ __device__ __forceinline__ void vt_fwd(double *re, double *im, double *xr, doubl
             if (s < 7) vt_cmul(cr, ci, z[1].x, z[1].y);
         }
     }
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        xr[VT_P1 * s + lane] = re[s];
-        xi[VT_P1 * s + lane] = im[s];
-    }
-    vh_wave_sync();
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        re[s] = xr[VT_P1 * hi + 8 * s + lo];
-        im[s] = xi[VT_P1 * hi + 8 * s + lo];
-    }
-    vh_wave_sync();
+    vt_exchange<SEQ>(re, im, xr, xi, lane, VT_P1, VT_P1 * hi + lo, 8);
     vt_dft8<-1>(re, im);
 #pragma unroll
     for (int s = 1; s < 8; s++) {
-        const double2 t = t2[(s - 1) * 8 + lo];
+        const double2 t = t2(s, lo);
         vt_cmul(re[s], im[s], t.x, t.y);
     }
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        xr[VT_P2 * lo + 8 * hi + s] = re[s];
-        xi[VT_P2 * lo + 8 * hi + s] = im[s];
-    }
-    vh_wave_sync();
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        re[s] = xr[VT_P2 * s + lane];
-        im[s] = xi[VT_P2 * s + lane];
-    }
-    vh_wave_sync();
+    vt_exchange<SEQ>(re, im, xr, xi, VT_P2 * lo + 8 * hi, 1, lane, VT_P2);
     vt_dft8<-1>(re, im);
 }
 
 // Inverse transform (unscaled): layout C in, layout A out.
+template <bool SEQ = false, typename T2>
 __device__ __forceinline__ void vt_inv(double *re, double *im, double *xr, double *xi, const double2 (&z)[2],
-                                       const double2 *t2, int lane)
+                                       const T2 &t2, int lane)
 {
     const int hi = lane >> 3, lo = lane & 7;
     vt_dft8<1>(re, im);
 #pragma unroll
     for (int s = 1; s < 8; s++) {
-        const double2 t = t2[(s - 1) * 8 + lo];
+        const double2 t = t2(s, lo);
         vt_cmul(re[s], im[s], t.x, -t.y);
     }
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        xr[VT_P2 * s + lane] = re[s];
-        xi[VT_P2 * s + lane] = im[s];
-    }
-    vh_wave_sync();
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        re[s] = xr[VT_P2 * lo + 8 * hi + s];
-        im[s] = xi[VT_P2 * lo + 8 * hi + s];
-    }
-    vh_wave_sync();
+    vt_exchange<SEQ>(re, im, xr, xi, lane, VT_P2, VT_P2 * lo + 8 * hi, 1);
     vt_dft8<1>(re, im);
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        xr[VT_P1 * hi + 8 * s + lo] = re[s];
-        xi[VT_P1 * hi + 8 * s + lo] = im[s];
-    }
-    vh_wave_sync();
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        re[s] = xr[VT_P1 * s + lane];
-        im[s] = xi[VT_P1 * s + lane];
-    }
-    vh_wave_sync();
+    vt_exchange<SEQ>(re, im, xr, xi, VT_P1 * hi + lo, 8, lane, VT_P1);
     {
         double cr = z[0].x, ci = z[0].y;
 #pragma unroll
@@ -284,6 +278,14 @@ __device__ __forceinline__ uint32_t vt_rot(const uint32_t *p, int j, uint32_t a)
     return (v ^ neg) - neg;
 }
 
+// add + coefficient j of X^a p, t = 4 (j - a): p[(j - a) mod N], negated when bit 10 of j - a is set
+__device__ __forceinline__ uint32_t vt_diff(const uint32_t *p, uint32_t t, uint32_t add)
+{
+    const uint32_t v = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(p) + (t & (4 * VT_N - 4)));
+    const uint32_t neg = (uint32_t)__builtin_amdgcn_sbfe((int)t, 12, 1);
+    return (v ^ neg) + (add - neg);
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -306,7 +308,7 @@ __global__ void __launch_bounds__(256) k_torus_fft(const uint32_t *__restrict__ 
     vt_lane_roots(z, t1, lane);
     double re[8], im[8];
     vt_fold(re, im, in + poly * VT_N, lane);
-    vt_fwd(re, im, lds[w][0], lds[w][1], z, t2, lane);
+    vt_fwd(re, im, lds[w][0], lds[w][1], z, vt_t2_lds{t2}, lane);
     double2 *o = out + poly * VT_M;
     const double scale = natural ? 1.0 : 1.0 / VT_M;
 #pragma unroll
@@ -325,18 +327,166 @@ hipError_t vh_launch_torus_fft(hipStream_t st, const uint32_t *in, double2 *out,
 }
 
 // ---------------------------------------------------------------------------
-// Blind rotation + extraction: one workgroup of two waves per LWE sample; wave c owns
-// component c of the accumulator (0: the mask a, 1: the body b), kept in LDS as
-// 32-bit words.  Per key index i with a non-zero amount:
-//   diff = X^a_i * acc_c - acc_c  (registers, 16 coefficients per lane)
-//   for each level l: digit polynomial -> forward transform -> accumulate its products
-//     with key rows (c * ell + l, output component 0 and 1) into two partial sums;
-//   the waves swap the partial of the other's component through LDS (two barriers),
-//   so wave c holds the sum over all 2 * ell rows for its component in a fixed order
-//   (wave 0's rows, then wave 1's); inverse transform, untwist (the key rows carry
-//   the 1/M of the inverse), round, and add into acc_c.
+// Blind rotation + extraction, one workgroup per LWE sample.  Per key index with a
+// non-zero amount, for each component c of the accumulator (0: the mask a, 1: the body b)
+// and level l: digit polynomial of X^a_i acc_c - acc_c -> forward transform -> products with
+// key row (c ell + l), output components 0 and 1; the products of all rows are summed per
+// output component, inverse transform, untwist (the key rows carry the 1/M of the inverse),
+// round, add into the accumulator.
+//
+// Few samples (k_torus_blind_rotate_wide): 2 ELL waves, one forward transform each.  Wave o < 2
+// also owns component o: its accumulator in registers, the digit forming and the inverse
+// transform.  acc[o] in LDS is wave o's own copy for the rotated reads, then holds the offset
+// difference y every wave takes its level's digits from.  Each wave writes its partial product
+// of a component it does not own to `area`; the owner adds them in wave order.  Before that a
+// wave's area is its exchange slice, and the owner's inverse exchanges run through an area it
+// has just read.  So an index takes two barriers: y in place, partials in place.
 // The key: n x (2 ell rows) x (2 components) x [slot][lane] double2 (layout C).
 // ---------------------------------------------------------------------------
+template <int ELL>   // levels (1..4)
+__global__ void __launch_bounds__(128 * ELL, 2) k_torus_blind_rotate_wide(vt_br_args A)
+{
+    constexpr int NW = 2 * ELL;
+    __shared__ uint32_t acc[2][VT_N];
+    __shared__ double2 area[2 * (NW - 1)][VT_M];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int l = w >> 1, mine = w == 1;   // level (of component w & 1); the component an owner wave keeps
+    const uint64_t k = blockIdx.x;
+    const uint32_t *in = A.lwe + k * (uint64_t)(A.n + 1);
+    const uint32_t two_n = 2 * VT_N;
+    const int shift = 32 - 11;   // log2(2^32 / 2N)
+    // partial product of component o by wave v (v != o)
+    auto part = [&](int o, int v) -> double2 * { return area[o * (NW - 1) + (v < o ? v : v - 1)]; };
+    double *xs = reinterpret_cast<double *>(part(w == 0 ? 1 : 0, w));
+    double *xi = reinterpret_cast<double *>(part(w & 1, NW - 1 - (w & 1) * (NW == 2)));   // read by wave w < 2 only
+    vt_t2_reg t2;
+#pragma unroll
+    for (int s = 0; s < 8; s++) t2.t[s] = A.consts[512 + 8 * s + (lane & 7)];
+    double2 z[2];
+    vt_lane_roots(z, A.consts, lane);
+
+    // acc = (0, X^-rot_b * tv): rot_b from b + floor(2^32 / (4 torus_base)) (cggi16.py:60-71)
+    const uint32_t rot_b = vt_mod_switch((uint64_t)in[A.n] + A.offset, shift, two_n);
+    const uint32_t rot_tv = (two_n - rot_b) & (two_n - 1);
+    uint32_t own[16];   // coefficients 64 s + lane of component w
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+        own[s] = w == 1 ? vt_rot(A.tv, 64 * s + lane, rot_tv) : 0u;
+        if (w < 2) acc[w][64 * s + lane] = own[s];
+    }
+
+    // Digits: with y = x + dec_off, field_l = (y >> sh_l) mod 2^B and d_l = field_l - 2^(B-1),
+    // which is the B-bit sign extension of field_l ^ 2^(B-1): one xor per coefficient, then
+    // one signed bit-field extract per level.
+    const uint32_t B = A.base_log;
+    uint32_t xmask = 0;
+#pragma unroll
+    for (int e = 1; e <= ELL; e++) xmask |= (1u << (B - 1)) << (32 - B * e);
+    const uint32_t sh = 32 - B * (l + 1);
+    uint32_t next = in[0];
+    for (uint32_t i = 0; i < A.n; i++) {
+        const uint32_t ai = vt_mod_switch(next, shift, two_n);
+        next = in[i + 1];   // the last one is the body
+        if (ai == 0) continue;
+        if (w < 2) {
+            // coefficient j of X^a acc: acc[(j - a) mod N], negated when bit 10 of j - a is set
+            const char *rows = reinterpret_cast<const char *>(acc[w]);
+            const uint32_t t0 = 4 * ((uint32_t)lane - ai);
+            uint32_t y[16];
+            vh_wave_sync();
+#pragma unroll
+            for (int s = 0; s < 16; s++) {
+                const uint32_t t = t0 + 256 * s;
+                const uint32_t v = *reinterpret_cast<const uint32_t *>(rows + (t & (4 * VT_N - 4)));
+                const uint32_t neg = (uint32_t)__builtin_amdgcn_sbfe((int)t, 12, 1);
+                y[s] = ((v ^ neg) + (A.dec_off - own[s] - neg)) ^ xmask;
+            }
+            vh_wave_sync();
+#pragma unroll
+            for (int s = 0; s < 16; s++) acc[w][64 * s + lane] = y[s];
+        }
+        __syncthreads();   // y of both components is in place
+        const VH_GLOBAL double *K = vh_global(reinterpret_cast<const double *>(
+            A.bsk + (((uint64_t)i * (2 * ELL) + (uint64_t)((w & 1) * ELL + l)) * 2) * VT_M + lane));
+        vh_f64x2 kw[8];
+        auto key = [&](int o) {   // the wave's key row, output component o
+#pragma unroll
+            for (int s = 0; s < 8; s++) kw[s] = *(const VH_GLOBAL vh_f64x2 *)(K + o * (2 * VT_M) + 128 * s);
+        };
+        key(1 - mine);   // lands during the transform
+        const uint32_t *yc = acc[w & 1];
+        double fr[8], fi[8];
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            fr[s] = (double)(int)__builtin_amdgcn_sbfe((int)yc[64 * s + lane], sh, B);
+            fi[s] = (double)(int)__builtin_amdgcn_sbfe((int)yc[64 * s + lane + VT_M], sh, B);
+        }
+        vt_slot_twist(fr, fi, false);
+        vt_fwd<true>(fr, fi, xs, nullptr, z, t2, lane);
+        vh_wave_sync();
+        double re[8], im[8];
+#pragma unroll
+        for (int oo = 0; oo < 2; oo++) {   // the other component's partial, then the own one
+            if (oo) key(mine);
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+                re[s] = __fma_rn(-fi[s], kw[s].y, fr[s] * kw[s].x);
+                im[s] = __fma_rn(fi[s], kw[s].x, fr[s] * kw[s].y);
+            }
+            if (oo == 0 || w >= 2) {
+                double2 *d = part(oo ? mine : 1 - mine, w) + lane;
+#pragma unroll
+                for (int s = 0; s < 8; s++) d[64 * s] = make_double2(re[s], im[s]);
+            }
+        }
+        __syncthreads();   // the partials are in place, y is read
+        if (w < 2) {
+#pragma unroll
+            for (int v = 1; v < NW; v++) {
+                const double2 *d = part(w, v - (v == 1 && w == 1)) + lane;   // waves other than w, ascending
+#pragma unroll
+                for (int s = 0; s < 8; s++) {
+                    const double2 p = d[64 * s];
+                    re[s] += p.x;
+                    im[s] += p.y;
+                }
+            }
+            vt_inv<true>(re, im, xi, nullptr, z, t2, lane);
+            vt_slot_twist(re, im, true);
+#pragma unroll
+            for (int s = 0; s < 8; s++) {   // the key carries the 1/M of the inverse
+                own[s] += vt_round_u32(re[s]);
+                own[s + 8] += vt_round_u32(im[s]);
+            }
+#pragma unroll
+            for (int s = 0; s < 16; s++) acc[w][64 * s + lane] = own[s];
+        }
+    }
+
+    if (w >= 2) return;
+    if (A.acc_out) {
+        uint32_t *o = A.acc_out + k * 2 * VT_N + (uint64_t)w * VT_N;
+#pragma unroll
+        for (int s = 0; s < 16; s++) o[64 * s + lane] = own[s];
+    }
+    if (A.out) {
+        // coefficient 0 of the phase b - a s: a'_0 = a_0, a'_j = -a_(N-j); b' = b_0
+        uint32_t *o = A.out + k * (VT_N + 1);
+        if (w == 0) {
+#pragma unroll
+            for (int s = 0; s < 16; s++) {
+                const int j = 64 * s + lane;
+                o[j ? VT_N - j : 0] = j ? 0u - own[s] : own[s];
+            }
+        } else if (lane == 0) {
+            o[VT_N] = own[0];
+        }
+    }
+}
+
+// Many samples: two waves, wave c owns component c of the accumulator (in LDS as 32-bit words)
+// and transforms its ELL digit polynomials one after another; the waves swap the partial
+// product of the other's component through LDS (two barriers).
 template <int ELL>   // levels (1..4)
 __global__ void __launch_bounds__(128, 2) k_torus_blind_rotate(vt_br_args A)
 {
@@ -373,11 +523,12 @@ __global__ void __launch_bounds__(128, 2) k_torus_blind_rotate(vt_br_args A)
         const uint32_t ai = vt_mod_switch(in[i], shift, two_n);
         if (ai == 0) continue;
         uint32_t dlo[8], dhi[8];
+        const uint32_t t0 = 4 * ((uint32_t)lane - ai);
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             const int j = 64 * s + lane;
-            dlo[s] = (vt_rot(mine, j, ai) - mine[j] + A.dec_off) ^ xmask;
-            dhi[s] = (vt_rot(mine, j + VT_M, ai) - mine[j + VT_M] + A.dec_off) ^ xmask;
+            dlo[s] = vt_diff(mine, t0 + 256 * s, A.dec_off - mine[j]) ^ xmask;
+            dhi[s] = vt_diff(mine, t0 + 256 * s + 4 * VT_M, A.dec_off - mine[j + VT_M]) ^ xmask;
         }
         // own: this wave's output component (w), other: the other wave's (1 - w)
         double por[8], poi[8], pxr[8], pxi[8];
@@ -402,7 +553,7 @@ __global__ void __launch_bounds__(128, 2) k_torus_blind_rotate(vt_br_args A)
                 im[s] = (double)(int)__builtin_amdgcn_sbfe((int)dhi[s], sh, B);
             }
             vt_slot_twist(re, im, false);
-            vt_fwd(re, im, xr, xi, z, t2, lane);
+            vt_fwd(re, im, xr, xi, z, vt_t2_lds{t2}, lane);
 #pragma unroll
             for (int s = 0; s < 8; s++) {
                 const double2 ko = kor[s], kx = kxr[s];
@@ -431,7 +582,7 @@ __global__ void __launch_bounds__(128, 2) k_torus_blind_rotate(vt_br_args A)
             im[s] = poi[s] + yi[s * 64 + lane];
         }
         __syncthreads();
-        vt_inv(re, im, xr, xi, z, t2, lane);
+        vt_inv(re, im, xr, xi, z, vt_t2_lds{t2}, lane);
         vt_slot_twist(re, im, true);
 #pragma unroll
         for (int s = 0; s < 8; s++) {   // the key carries the 1/M of the inverse
@@ -456,15 +607,21 @@ __global__ void __launch_bounds__(128, 2) k_torus_blind_rotate(vt_br_args A)
     }
 }
 
-hipError_t vh_launch_torus_blind_rotate(hipStream_t st, const vt_br_args &A, uint64_t count)
+hipError_t vh_launch_torus_blind_rotate(hipStream_t st, const vt_br_args &A, uint64_t count, unsigned cus)
 {
     if (!count) return hipSuccess;
-    switch (A.ell) {
-    case 1: VH_KL(k_torus_blind_rotate<1>, dim3((unsigned)count), dim3(128), 0, st, A); break;
-    case 2: VH_KL(k_torus_blind_rotate<2>, dim3((unsigned)count), dim3(128), 0, st, A); break;
-    case 3: VH_KL(k_torus_blind_rotate<3>, dim3((unsigned)count), dim3(128), 0, st, A); break;
-    case 4: VH_KL(k_torus_blind_rotate<4>, dim3((unsigned)count), dim3(128), 0, st, A); break;
-    default: return hipErrorInvalidValue;
-    }
+    // Up to one sample per CU the levels of both components run side by side: 3 samples at
+    // n = 630, 3 levels take 2.61 ms against 3.39 ms, 256 take 2.77 against 3.60.  From two samples
+    // per CU on the chip is full of FP64 work either way, and the two-wave form has less LDS
+    // traffic for the partial sums (400 samples: 5.1 ms; 1024: 6.2 ms).
+    const dim3 grid((unsigned)count);
+    const bool wide = count <= cus;
+#define VT_BR(EE)                                                                                       \
+    case EE:                                                                                            \
+        if (wide) VH_KL(k_torus_blind_rotate_wide<EE>, grid, dim3(128 * EE), 0, st, A);                 \
+        else VH_KL(k_torus_blind_rotate<EE>, grid, dim3(128), 0, st, A);                                \
+        break;
+    switch (A.ell) { VT_BR(1) VT_BR(2) VT_BR(3) VT_BR(4) default: return hipErrorInvalidValue; }
+#undef VT_BR
     return hipGetLastError();
 }
