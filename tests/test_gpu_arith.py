@@ -397,6 +397,51 @@ def test_ntt_mul_intt_batch(lib, N, L, count):
         pool.free(p)
 
 
+@pytest.mark.parametrize("N,widths,split", [
+    (256, (50, 60), 1),                  # below the register sizes: separate transforms
+    (512, (50,), 1), (512, (60, 49, 51), 1), (1024, (60,), 1), (2048, (50, 60), 1), (4096, (60, 50, 40), 1),
+    (8192, (60,), 1), (16384, (60, 50), 1), (32768, (51, 60), 1), (65536, (60, 50), 1),
+    (4096, (60, 62), 1), (8192, (62, 50), 1),   # a limb above 2^62: separate transforms
+    (4096, (49, 60), 4),                 # split degree 4: the wrap-aware product
+])
+def test_ntt_mul_intt_prime_widths(lib, N, widths, split):
+    """The product over every arithmetic and size class, limbs of one ring in different classes, an odd
+    batch (the last workgroup of small rows partly empty), largest residues in one pair, a limb mask
+    with a gap in another, against the oracle."""
+    n2, primes = 2 * N // split, []
+    for b in widths:   # above 2^50: the first prime past 2^b; else below
+        q = int(O.lib().o_next_special_prime(1 << b, N // split, 1)) if b > 50 else O.gen_prime(n2, b, primes)
+        primes.append(q)
+    count, L = 3, len(primes)
+    pool, c = rt.Pool(N, primes, split), O.Ctx(N, primes, split)
+    rng = np.random.default_rng(N + sum(widths))
+    masks = [(1 << L) - 1] * count
+    xs = [rt.random_rows(rng, primes, N) for _ in range(count)]
+    ys = [rt.random_rows(rng, primes, N) for _ in range(count)]
+    for i, q in enumerate(primes):
+        xs[1][i], ys[1][i] = q - 1, q - 1
+    if L > 2:
+        masks[2] = 0b101
+    px = [pool.poly(x, m) for x, m in zip(xs, masks)]
+    py, pz = [pool.poly(y) for y in ys], [pool.poly() for _ in range(count)]
+    print(f"[product] N={N} widths={widths} split={split}", flush=True)
+    lib.vfhe_hip_ntt_mul_intt_batch(rt._native.voidp_array(pz), rt._native.voidp_array(px),
+                                    rt._native.voidp_array(py), count)
+    for k in range(count):
+        a, b, z = np.zeros_like(xs[k]), np.zeros_like(xs[k]), np.zeros_like(xs[k])
+        c.to_ntt(a, xs[k], masks[k])
+        c.to_ntt(b, ys[k], masks[k])
+        c.mul(z, a, masks[k], b, masks[k], 0)
+        c.to_coeff(z, z, masks[k])
+        assert pool.mask(pz[k]) == masks[k]
+        got = pool.read(pz[k])
+        for i in range(L):
+            if (masks[k] >> i) & 1:
+                assert np.array_equal(got[i], z[i]), (k, i)
+    for p in px + py + pz:
+        pool.free(p)
+
+
 @pytest.mark.slow
 def test_ntt_mul_intt_batch64_config2(lib):
     """The benchmarked fused-product batch: 64 pairs at N = 2^16, L = 24 in one call.  Every product

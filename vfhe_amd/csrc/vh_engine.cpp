@@ -766,11 +766,16 @@ static int col_wide(unsigned items, int logn)
 }
 
 // Forward (dir 0) or inverse (dir 1) transforms of n-point rows.
+// Arithmetic of a limb's transform: FP64 below 2^50, lazy 64-bit residues below 2^62, canonical
+// 64-bit residues (the radix-2 kernel only) up to the engine's limit.
+enum { VH_NTT_WIDE = 0, VH_NTT_FP64 = 1, VH_NTT_INT = 2 };
+static int ntt_kind(const vh_limb &h) { return h.fp64 ? VH_NTT_FP64 : h.q < (1ULL << 62) ? VH_NTT_INT : VH_NTT_WIDE; }
+
 // Launches the transforms of `cnt` staged work items (device list d_items, all of one
-// arithmetic path: fp = FP64 limbs) of n-point rows, direction dir.
-static void ntt_dispatch(const vh_item *d_items, unsigned cnt, const vh_limb *d_limbs, int fp, uint64_t n, int dir)
+// arithmetic, ntt_kind) of n-point rows, direction dir.
+static void ntt_dispatch(const vh_item *d_items, unsigned cnt, const vh_limb *d_limbs, int kind, uint64_t n, int dir)
 {
-    const int logn = ilog2(n);
+    const int logn = ilog2(n), fp = kind == VH_NTT_FP64;
     if (fp && logn >= 13 && logn <= 16 && OPT.ntt_mode == 1 && C.xcd_ok) {
         // Persistent kernel: both passes of every transform on one XCD, the
         // intermediate exchanged through that XCD's L2.
@@ -812,11 +817,17 @@ static void ntt_dispatch(const vh_item *d_items, unsigned cnt, const vh_limb *d_
                 { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16(S(), ci, cc, d_limbs, 1, logn, 0, R1, 1, 0, 1)); }
             }
         }
-    } else if (fp && logn >= 9 && logn <= 12 && OPT.ntt_small) {
+    } else if (kind != VH_NTT_WIDE && logn >= 9 && logn <= 12 && OPT.ntt_small) {
         // whole transforms in registers, 4096/N of them per workgroup
-        vh_prof_scope ps_(VH_PROF_NTT_FP64);
-        VH_LAUNCH(vh_launch_ntt_small(S(), d_items, cnt, d_limbs, dir, logn));
+        vh_prof_scope ps_(fp ? VH_PROF_NTT_FP64 : VH_PROF_NTT_INT);
+        VH_LAUNCH(vh_launch_ntt_small(S(), d_items, cnt, d_limbs, dir, logn, fp));
         g_ntt_small_launches++;
+    } else if (kind == VH_NTT_INT && logn >= 13 && logn <= 16) {
+        // two register passes, column then row (inverse: row then column)
+        for (int pass = 0; pass < 2; pass++) {
+            vh_prof_scope ps_(VH_PROF_NTT_INT);
+            VH_LAUNCH(vh_launch_ntt16i(S(), d_items, cnt, d_limbs, dir, logn, pass == dir));
+        }
     } else if (logn <= 12) {
         { vh_prof_scope ps_(fp ? VH_PROF_NTT_FP64 : VH_PROF_NTT_INT); VH_LAUNCH(vh_launch_ntt_pass(S(), d_items, cnt, d_limbs, fp, dir, logn, 0, logn, 0, 1, 1, 1)); }
     } else {
@@ -837,17 +848,17 @@ static void ntt_dispatch(const vh_item *d_items, unsigned cnt, const vh_limb *d_
 static void run_ntt(std::vector<vh_item> &items, const vh_limb *d_limbs, const vh_limb *h_limbs, uint64_t n, int dir)
 {
     if (items.empty()) return;
-    std::vector<vh_item> grp[2];
-    for (auto &it : items) grp[h_limbs[it.limb].fp64 ? 1 : 0].push_back(it);
+    std::vector<vh_item> grp[3];
+    for (auto &it : items) grp[ntt_kind(h_limbs[it.limb])].push_back(it);
     // Limb-major order: workgroups running together share one limb's twiddle table in L2.
     for (auto &g : grp)
         std::stable_sort(g.begin(), g.end(), [](const vh_item &a, const vh_item &b) { return a.limb < b.limb; });
-    for (int fp = 0; fp < 2; fp++) {
-        auto &v = grp[fp];
+    for (int kind = 0; kind < 3; kind++) {
+        auto &v = grp[kind];
         for (size_t off = 0; off < v.size(); off += VH_MAX_GRID_Y) {
             const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, v.size() - off);
             std::vector<vh_item> chunk(v.begin() + off, v.begin() + off + cnt);
-            ntt_dispatch(vh_stage_vec(chunk), cnt, d_limbs, fp, n, dir);
+            ntt_dispatch(vh_stage_vec(chunk), cnt, d_limbs, kind, n, dir);
         }
     }
 }
@@ -3268,8 +3279,13 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
     vh_pool *P = VPOOL(t);
     const uint64_t nd = Cc * J.size(), next = E.size();
     bool fp = true;   // FP64 limbs only: the lift folds into the NTT and the inner product runs in FP64
-    for (int e : E) fp = fp && P->h_limbs[e].fp64;
-    for (int j : J) fp = fp && P->h_limbs[j].fp64;
+    bool lazy = true;
+    for (const auto *list : {&E, &J})
+        for (int e : *list) {
+            fp = fp && P->h_limbs[e].fp64;
+            lazy = lazy && ntt_kind(P->h_limbs[e]) == VH_NTT_INT;
+        }
+    const int kind = fp ? VH_NTT_FP64 : lazy ? VH_NTT_INT : VH_NTT_WIDE;
     if (fp && OPT.br_fused && N == 1024 && Cc <= 2 && divs.size() == 1 && J.size() <= VH_BR_MAXJ &&
         next == J.size() + 1) {
         // Every key index in one launch, each accumulator resident in its workgroup's LDS.
@@ -3468,7 +3484,7 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
             vh_prof_scope ps_(VH_PROF_ELTWISE);
             VH_LAUNCH(vh_launch_eltwise(S(), d_lift + off, cn, P->d_limbs, VH_OP_REDUCE, N));
         });
-        chunks(nt.size(), [&](size_t off, unsigned cn) { ntt_dispatch(d_nt + off, cn, P->d_limbs, fp, N, 0); });
+        chunks(nt.size(), [&](size_t off, unsigned cn) { ntt_dispatch(d_nt + off, cn, P->d_limbs, kind, N, 0); });
         // 3. external product with bk[i]: row (ti, d, c) of the key table
         for (uint64_t d = 0; d < nd; d++) {
             const uint64_t src = d / J.size(), jj = d % J.size();
@@ -3486,7 +3502,7 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
             VH_LAUNCH(vh_launch_keyswitch_mac(S(), d_jobs + off, cn, (unsigned)next, P->d_limbs, d_kptr, N, fp ? 1 : 0));
         });
         // 4. back to coefficient form, round-divided by the special limbs (their rows cleared)
-        chunks(inv.size(), [&](size_t off, unsigned cn) { ntt_dispatch(d_inv + off, cn, P->d_limbs, fp, N, 1); });
+        chunks(inv.size(), [&](size_t off, unsigned cn) { ntt_dispatch(d_inv + off, cn, P->d_limbs, kind, N, 1); });
         if (!divs.empty()) {
             chunks(dj.size(), [&](size_t off, unsigned cn) {
                 vh_prof_scope ps_(VH_PROF_DIVISION);
@@ -3816,12 +3832,11 @@ extern "C" int vfhe_hip_ntt_batch_noalloc(RNS_Polynomial *polys, uint64_t count,
     return 0;
 }
 
-// The fused product's three launches (N = 2^13..2^16, FP64 limbs): forward column
-// passes of x into z and of y into its temporary row (col), forward row stages of
-// both, pointwise product and inverse row stages in one kernel (mid), inverse
-// column pass (inv).
+// The fused product's three launches (N = 2^13..2^16), FP64 or lazy integer limbs: forward column
+// passes of x into z and of y into its temporary row (col), forward row stages of both, pointwise
+// product and inverse row stages in one kernel (mid), inverse column pass (inv).
 static void fused_product_launches(std::vector<vh_item> &col, std::vector<vh_item> &mid, std::vector<vh_item> &inv,
-                                   const vh_pool *P, int logn)
+                                   const vh_pool *P, int logn, int kind)
 {
     const int R1 = logn - 8;
     auto launch = [&](std::vector<vh_item> &v, int which) {
@@ -3829,6 +3844,12 @@ static void fused_product_launches(std::vector<vh_item> &col, std::vector<vh_ite
             const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, v.size() - off);
             std::vector<vh_item> chunk(v.begin() + off, v.begin() + off + cnt);
             const vh_item *d = vh_stage_vec(chunk);
+            if (kind == VH_NTT_INT) {
+                vh_prof_scope ps_(VH_PROF_NTT_INT);
+                if (which == 1) VH_LAUNCH(vh_launch_ntt16i_row_mul(S(), d, cnt, P->d_limbs, logn));
+                else VH_LAUNCH(vh_launch_ntt16i(S(), d, cnt, P->d_limbs, which == 0 ? 0 : 1, logn, 1));
+                continue;
+            }
             vh_prof_scope ps_(VH_PROF_NTT_FP64);
             const bool pipe = OPT.ntt_mode == 2 && C.pipe_blocks > 0;
             const unsigned nb0 = (OPT.ntt_tile_grid & 1) ? UINT_MAX : C.pipe_blocks;
@@ -3847,73 +3868,88 @@ static void fused_product_launches(std::vector<vh_item> &col, std::vector<vh_ite
     launch(inv, 2);
 }
 
+// Every product of one batch: whole rows in one kernel (N = 2^9..2^12), three launches (N =
+// 2^13..2^16), or separate transforms and products (other sizes, split rings, limbs above 2^62, the
+// persistent schedule).  Temporary rows of a batch come from one block.
 static void ntt_mul_intt(RNS_Polynomial *z, RNS_Polynomial *x, RNS_Polynomial *y, uint64_t count)
 {
     incNTT t = z[0]->ntt;
-    const uint64_t N = t->N;
-    std::vector<RNS_Polynomial> tmp(count);
-    std::vector<vh_mulreq> muls;
+    const uint64_t N = t->N, split = t->split_degree;
+    vh_pool *P = VPOOL(t);
+    const int logn = ilog2(P->n);
+    uint64_t rows = 0;
+    bool kinds[3] = {false, false, false};
     for (uint64_t i = 0; i < count; i++) {
         VH_REQUIRE(z[i] != x[i] && z[i] != y[i]);
         dev_ready(x[i]); dev_ready(y[i]); dev_ready(z[i]);
         const uint64_t m = x[i]->rns_mask & y[i]->rns_mask;
         check_rows(z[i], m);
-        tmp[i] = new_poly(N, m, t, false, false);
         z[i]->rns_mask = m;
+        for_active(m, t->l, [&](uint64_t li) { rows++; kinds[ntt_kind(P->h_limbs[li])] = true; });
     }
-    vh_pool *P = VPOOL(t);
-    const int logn = ilog2(P->n);
-    bool fused = t->split_degree == 1 && OPT.ntt_mode != 1 && logn >= 13 && logn <= 16;
-    for (uint64_t i = 0; i < count && fused; i++)
-        for_active(z[i]->rns_mask, t->l, [&](uint64_t li) { fused = fused && P->h_limbs[li].fp64; });
-    if (fused) {
-        // Three launches: forward column passes of x (into z) and y (into tmp); forward
-        // row stages, product and inverse row stages in one kernel; inverse column pass.
-        // Items limb-major: the pipelined passes reload their twiddle table head when the
-        // limb changes.
-        std::vector<vh_item> col, mid, inv;
+    if (!rows) return;
+    const bool small = split == 1 && logn >= 9 && logn <= 12 && OPT.ntt_small && !kinds[VH_NTT_WIDE];
+    const bool fused = split == 1 && logn >= 13 && logn <= 16 && OPT.ntt_mode != 1 && !kinds[VH_NTT_WIDE];
+    // Items limb-major: workgroups in flight share one limb's twiddles.
+    auto each = [&](int kind, const std::function<void(uint64_t, uint64_t)> &f) {
         for (uint64_t li = 0; li < t->l; li++)
-            for (uint64_t i = 0; i < count; i++) {
-                if (!((z[i]->rns_mask >> li) & 1)) continue;
-                col.push_back(mk_item(drow(x[i], li), drow(z[i], li), (uint32_t)li));
-                col.push_back(mk_item(drow(y[i], li), drow(tmp[i], li), (uint32_t)li));
-                mid.push_back(mk_item(drow(z[i], li), drow(z[i], li), (uint32_t)li, drow(tmp[i], li)));
-                inv.push_back(mk_item(drow(z[i], li), drow(z[i], li), (uint32_t)li));
+            for (uint64_t i = 0; i < count; i++)
+                if (((z[i]->rns_mask >> li) & 1) && (kind < 0 || ntt_kind(P->h_limbs[li]) == kind)) f(i, li);
+    };
+    if (small) {
+        for (int kind : {VH_NTT_FP64, VH_NTT_INT}) {
+            std::vector<vh_item> items;
+            each(kind, [&](uint64_t i, uint64_t li) { items.push_back(mk_item(drow(x[i], li), drow(z[i], li), (uint32_t)li, drow(y[i], li))); });
+            for (size_t off = 0; off < items.size(); off += VH_MAX_GRID_Y) {
+                const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, items.size() - off);
+                std::vector<vh_item> chunk(items.begin() + off, items.begin() + off + cnt);
+                vh_prof_scope ps_(kind == VH_NTT_FP64 ? VH_PROF_NTT_FP64 : VH_PROF_NTT_INT);
+                VH_LAUNCH(vh_launch_product_small(S(), vh_stage_vec(chunk), cnt, P->d_limbs, logn, kind == VH_NTT_FP64));
             }
-        fused_product_launches(col, mid, inv, P, logn);
-        for (auto p : tmp) free_RNS_polynomial(p);
+        }
         return;
     }
-    {
-        // forward transforms of x into z and of y into a temporary, common limbs only
-        std::vector<vh_item> items;
-        for (uint64_t i = 0; i < count; i++) {
-            const uint64_t m = z[i]->rns_mask;
-            for_active(m, t->l, [&](uint64_t li) {
-                for (uint64_t k = 0; k < t->split_degree; k++) {
-                    items.push_back(mk_item(drow(x[i], li) + k * P->n, drow(z[i], li) + k * P->n, (uint32_t)li));
-                    items.push_back(mk_item(drow(y[i], li) + k * P->n, drow(tmp[i], li) + k * P->n, (uint32_t)li));
-                }
+    uint64_t *tmp = (uint64_t *)vh_dmalloc((split > 1 ? 2 : 1) * rows * N * 8), r = 0;
+    if (fused) {
+        for (int kind : {VH_NTT_FP64, VH_NTT_INT}) {
+            std::vector<vh_item> col, mid, inv;
+            each(kind, [&](uint64_t i, uint64_t li) {
+                uint64_t *ty = tmp + r++ * N, *zr = drow(z[i], li);
+                col.push_back(mk_item(drow(x[i], li), zr, (uint32_t)li));
+                col.push_back(mk_item(drow(y[i], li), ty, (uint32_t)li));
+                mid.push_back(mk_item(zr, zr, (uint32_t)li, ty));
+                inv.push_back(mk_item(zr, zr, (uint32_t)li));
             });
+            if (!col.empty()) fused_product_launches(col, mid, inv, P, logn, kind);
         }
-        run_ntt(items, P->d_limbs, P->h_limbs.data(), P->n, 0);
+        vh_dfree(tmp);
+        return;
     }
-    for (uint64_t i = 0; i < count; i++) muls.push_back({z[i], z[i], tmp[i], z[i]->rns_mask});
-    if (t->split_degree == 1) {
-        run_muls(muls, 0);
+    // forward transforms of x and y, the products, the inverse transforms.  The wrap-aware product of
+    // a split ring needs operands distinct from its output.
+    std::vector<vh_item> fwd, mul, inv;
+    each(-1, [&](uint64_t i, uint64_t li) {
+        uint64_t *zr = drow(z[i], li), *ty = tmp + r++ * N, *tx = split > 1 ? tmp + r++ * N : zr;
+        for (uint64_t k = 0; k < split; k++) {
+            fwd.push_back(mk_item(drow(x[i], li) + k * P->n, tx + k * P->n, (uint32_t)li));
+            fwd.push_back(mk_item(drow(y[i], li) + k * P->n, ty + k * P->n, (uint32_t)li));
+            inv.push_back(mk_item(zr + k * P->n, zr + k * P->n, (uint32_t)li));
+        }
+        mul.push_back(mk_item(tx, zr, (uint32_t)li, ty, split > 1 ? (uint64_t)(uintptr_t)P->d_w[li] : 0, 0, (uint32_t)split));
+    });
+    run_ntt(fwd, P->d_limbs, P->h_limbs.data(), P->n, 0);
+    if (split == 1) {
+        run_eltwise(mul, P->d_limbs, VH_OP_MUL, N);
     } else {
-        // the wrap-aware product needs an operand distinct from its output
-        for (uint64_t i = 0; i < count; i++) {
-            RNS_Polynomial zz = polynomial_new_RNS_polynomial(N, z[i]->rns_mask, t);
-            copy_rows(zz, z[i], z[i]->rns_mask);
-            run_muls({{z[i], zz, tmp[i], z[i]->rns_mask}}, 0);
-            free_RNS_polynomial(zz);
+        for (size_t off = 0; off < mul.size(); off += VH_MAX_GRID_Y) {
+            const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, mul.size() - off);
+            std::vector<vh_item> chunk(mul.begin() + off, mul.begin() + off + cnt);
+            vh_prof_scope ps_(VH_PROF_ELTWISE);
+            VH_LAUNCH(vh_launch_split_mul(S(), vh_stage_vec(chunk), cnt, P->d_limbs, 0, P->n, split));
         }
     }
-    std::vector<std::pair<RNS_Polynomial, RNS_Polynomial>> inv;
-    for (uint64_t i = 0; i < count; i++) inv.push_back({z[i], z[i]});
-    ntt_rows(inv, 1);
-    for (auto p : tmp) free_RNS_polynomial(p);
+    run_ntt(inv, P->d_limbs, P->h_limbs.data(), P->n, 1);
+    vh_dfree(tmp);
 }
 
 extern "C" void vfhe_hip_ntt_mul_intt_batch(RNS_Polynomial *z, RNS_Polynomial *x, RNS_Polynomial *y, uint64_t count)

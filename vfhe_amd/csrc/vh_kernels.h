@@ -89,9 +89,18 @@ struct vh_mac_job {
     uint64_t pass_mask;
 };
 
-// Whole FP64 transforms of N = 2^9 .. 2^12 (reads it.src, writes it.dst), registers radix-16.
+// Whole transforms of N = 2^9 .. 2^12 (reads it.src, writes it.dst), and whole negacyclic products
+// z = INTT(NTT(x) NTT(y)) (x it.src, y it.src2, z it.dst), in registers.  fp: every limb FP64,
+// else every limb integer with q < 2^62.
 hipError_t vh_launch_ntt_small(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, int dir,
-                               int logn);
+                               int logn, int fp);
+hipError_t vh_launch_product_small(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs,
+                                   int logn, int fp);
+// Integer path (q < 2^62), N = 2^13 .. 2^16: one pass of a transform (dir 0: col then row, dir 1: row
+// then col; the first pass reads it.src, the second works in it.dst), and the product's middle step.
+hipError_t vh_launch_ntt16i(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, int dir,
+                            int logn, int col);
+hipError_t vh_launch_ntt16i_row_mul(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, int logn);
 // Fused CGGI blind rotation (N = 1024, FP64 limbs, one special prime): accumulator k steps
 // through every key index with its rows in its workgroup's registers and LDS; waves 2w and
 // 2w + 1 of an accumulator work modulo extended limb E[w].

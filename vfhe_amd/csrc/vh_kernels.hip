@@ -1459,150 +1459,6 @@ static inline unsigned vh_blocks(uint64_t n, unsigned per = 256, unsigned cap = 
 }
 
 // ---------------------------------------------------------------------------
-// Whole transforms of N = 2^9 .. 2^12 points on the FP64 path, 16 values per thread in
-// registers: T = N/16 threads per transform, 4096/N transforms per 256-thread workgroup.
-// The reference's butterfly network (merged CT forward, natural in, bit-reversed out;
-// GS inverse with n^-1, ntt.c / ntt50.c) in three register phases:
-//   A  stages 0..3         stride ownership   j = t + T m            (uniform twiddles)
-//   B  stages 4..7         middle ownership   j = 16U g + u + U m    (t = u + U g, U = T/16)
-//   C  stages 8..logN-1    contiguous         j = 16 t + m
-// with an LDS exchange between phases (one pad slot per 16 values: the contiguous reads
-// stride 17 words).  A stage-s butterfly on (j, j + N/2^(s+1)) takes the twiddle of index
-// 2^s + (j >> (logN - s)), so every product is the reference's and the canonical outputs
-// are identical.  Rows are loaded and stored in the stride ownership (whole 128-byte runs
-// per instruction); the forward pass regroups its output through LDS for that.
-// Bounds as in the two-pass kernels: at most four stages between centrings, |x| < 2^52.
-// ---------------------------------------------------------------------------
-// Register cores of the transform for T = N/16 threads (thread index t < T); lds holds
-// N + N/16 doubles private to the transform.  WAVE: the transform's threads are one wave
-// (or part of one), so the exchanges need only the wave's own ordering.
-template <int LOGN> struct vh_reg_ntt {
-    static constexpr int N = 1 << LOGN, T = N / 16, U = T / 16;
-    static __device__ __forceinline__ int li(int j) { return j + (j >> 4); }
-    static __device__ __forceinline__ int jA(int t, int m) { return t + T * m; }
-    static __device__ __forceinline__ int jB(int t, int m) { return 16 * U * (t / U) + t % U + U * m; }
-    static __device__ __forceinline__ int jC(int t, int m) { return 16 * t + m; }
-    template <bool WAVE> static __device__ __forceinline__ void sync()
-    {
-        if (WAVE) vh_wave_sync();
-        else __syncthreads();
-    }
-    template <bool WAVE, typename FW, typename FR>
-    static __device__ __forceinline__ void exchange(double (&v)[16], double *lds, FW jw, FR jr, bool centre, double q,
-                                                    double qinv)
-    {
-#pragma unroll
-        for (int m = 0; m < 16; m++) lds[li(jw(m))] = centre ? vh_center(v[m], q, qinv) : v[m];
-        sync<WAVE>();
-#pragma unroll
-        for (int m = 0; m < 16; m++) v[m] = lds[li(jr(m))];
-        sync<WAVE>();
-    }
-    // forward: v in the stride ownership (any |v| < 2^51) -> contiguous ownership, |v| < 2^52
-    template <bool WAVE>
-    static __device__ __forceinline__ void fwd(double (&v)[16], double *lds, int t, const VH_GLOBAL double *tw,
-                                               double q, double qinv)
-    {
-        const int g = t / U;
-        auto ct = [&](int s, int hm, auto blk) {
-#pragma unroll
-            for (int m = 0; m < 16; m++) {
-                if (m & hm) continue;
-                const int i = (1 << s) + blk(m);
-                const double x = vh_mulmod_tw(v[m + hm], tw[2 * i], tw[2 * i + 1], q);
-                const double a = v[m];
-                v[m] = a + x;
-                v[m + hm] = a - x;
-            }
-        };
-#pragma unroll
-        for (int s = 0; s < 4; s++) ct(s, 8 >> s, [&](int m) { return m >> (4 - s); });
-        exchange<WAVE>(v, lds, [&](int m) { return jA(t, m); }, [&](int m) { return jB(t, m); }, true, q, qinv);
-#pragma unroll
-        for (int s = 4; s < 8; s++) ct(s, 8 >> (s - 4), [&](int m) { return (g << (s - 4)) + (m >> (8 - s)); });
-        exchange<WAVE>(v, lds, [&](int m) { return jB(t, m); }, [&](int m) { return jC(t, m); }, true, q, qinv);
-#pragma unroll
-        for (int s = 8; s < LOGN; s++) ct(s, 1 << (LOGN - s - 1), [&](int m) { return (16 * t + m) >> (LOGN - s); });
-    }
-    // inverse (before the n^-1 factor): v in the contiguous ownership (|v| <= q) -> stride
-    // ownership, |v| < 2^52; GS sums re-centred after every second stage
-    template <bool WAVE>
-    static __device__ __forceinline__ void inv(double (&v)[16], double *lds, int t, const VH_GLOBAL double *tw,
-                                               double q, double qinv)
-    {
-        const int g = t / U;
-        int c = 0;
-        auto gs = [&](int s, int hm, auto blk) {
-#pragma unroll
-            for (int m = 0; m < 16; m++) {
-                if (m & hm) continue;
-                const int i = (1 << s) + blk(m);
-                const double a = v[m], x = v[m + hm];
-                double sum = a + x;
-                if (c & 1) sum = vh_center(sum, q, qinv);
-                v[m] = sum;
-                v[m + hm] = vh_mulmod_tw(a - x, tw[2 * i], tw[2 * i + 1], q);
-            }
-            c++;
-        };
-#pragma unroll
-        for (int s = LOGN - 1; s >= 8; s--) gs(s, 1 << (LOGN - s - 1), [&](int m) { return (16 * t + m) >> (LOGN - s); });
-        exchange<WAVE>(v, lds, [&](int m) { return jC(t, m); }, [&](int m) { return jB(t, m); }, false, q, qinv);
-#pragma unroll
-        for (int s = 7; s >= 4; s--) gs(s, 8 >> (s - 4), [&](int m) { return (g << (s - 4)) + (m >> (8 - s)); });
-        exchange<WAVE>(v, lds, [&](int m) { return jB(t, m); }, [&](int m) { return jA(t, m); }, false, q, qinv);
-#pragma unroll
-        for (int s = 3; s >= 0; s--) gs(s, 8 >> s, [&](int m) { return m >> (4 - s); });
-    }
-};
-
-template <int DIR, int LOGN>
-__global__ void __launch_bounds__(256)
-k_ntt_small(const vh_item *__restrict__ items, unsigned nitems, const vh_limb *__restrict__ limbs)
-{
-    using R = vh_reg_ntt<LOGN>;
-    constexpr int N = R::N, T = R::T, PER = 256 / T, PAD = N + N / 16;
-    constexpr bool WAVE = T <= 64;
-    static_assert(LOGN >= 9 && LOGN <= 12, "k_ntt_small: N = 2^9 .. 2^12");
-    __shared__ double lds_all[PER * PAD];
-    const int tid = threadIdx.x, slot = tid / T, t = tid % T;
-    const unsigned idx = blockIdx.x * PER + slot;
-    const bool live = idx < nitems;
-    // a slot past the end transforms the last item again (every thread reaches the
-    // barriers) and stores nothing
-    const vh_item &it = items[live ? idx : nitems - 1];
-    const vh_limb &L = limbs[it.limb];
-    const double q = L.qd, qinv = L.qinv;
-    const VH_GLOBAL double *tw = vh_global(reinterpret_cast<const double *>(DIR == 0 ? L.tw_fwd : L.tw_inv));
-    double *lds = lds_all + slot * PAD;
-    const VH_GLOBAL uint64_t *in = vh_global(it.src);
-    VH_GLOBAL uint64_t *out = vh_global(it.dst);
-    double v[16];
-#pragma unroll
-    for (int m = 0; m < 16; m++) v[m] = vh_u2d(vh_ld(in + R::jA(t, m)));
-    if (DIR == 0) {
-        R::template fwd<WAVE>(v, lds, t, tw, q, qinv);
-#pragma unroll
-        for (int m = 0; m < 16; m++) v[m] = __longlong_as_double((long long)vh_d2u(vh_canon(v[m], q, qinv)));
-        R::template exchange<WAVE>(v, lds, [&](int m) { return R::jC(t, m); }, [&](int m) { return R::jA(t, m); },
-                                   false, q, qinv);
-        if (live) {
-#pragma unroll
-            for (int m = 0; m < 16; m++) vh_st(out + R::jA(t, m), (uint64_t)__double_as_longlong(v[m]));
-        }
-    } else {
-        R::template exchange<WAVE>(v, lds, [&](int m) { return R::jA(t, m); }, [&](int m) { return R::jC(t, m); },
-                                   false, q, qinv);
-        R::template inv<WAVE>(v, lds, t, tw, q, qinv);
-        if (live) {
-#pragma unroll
-            for (int m = 0; m < 16; m++)
-                vh_st(out + R::jA(t, m), vh_d2u(vh_canon(vh_mulmod_tw(v[m], L.ninv_d, L.ninv_q, q), q, qinv)));
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Batched sample extraction: one thread per output word (grid-stride).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_extract_lwe(const uint64_t *const *__restrict__ src,
@@ -1699,21 +1555,6 @@ __global__ void __launch_bounds__(256) k_alu_rate(int kind, int iters, uint64_t 
 hipError_t vh_launch_alu_rate(hipStream_t st, int kind, int iters, unsigned blocks, uint64_t *out)
 {
     VH_KL(k_alu_rate, dim3(blocks), dim3(256), 0, st, kind, iters, out);
-    return hipGetLastError();
-}
-
-hipError_t vh_launch_ntt_small(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, int dir,
-                               int logn)
-{
-    if (logn < 9 || logn > 12 || nitems == 0) return hipErrorInvalidValue;
-    const unsigned per = 4096u >> logn, nb = (nitems + per - 1) / per;
-#define VH_SMALL(LG)                                                                                        \
-    if (logn == LG) {                                                                                       \
-        if (dir == 0) VH_KL((k_ntt_small<0, LG>), dim3(nb), dim3(256), 0, st, items, nitems, limbs);         \
-        else VH_KL((k_ntt_small<1, LG>), dim3(nb), dim3(256), 0, st, items, nitems, limbs);                  \
-    }
-    VH_SMALL(9) VH_SMALL(10) VH_SMALL(11) VH_SMALL(12)
-#undef VH_SMALL
     return hipGetLastError();
 }
 
