@@ -208,6 +208,35 @@ def test_moddown_rescale_fp64_against_integer_and_oracle(lib, K):
     s.check(got[1][0], ref, m2)
 
 
+@pytest.mark.parametrize("N,L,K,batch", [(256, 3, 1, 300), (256, 2, 2, 3), (4096, 5, 3, 2), (1024, 4, 4, 150), (16, 1, 1, 3)])
+def test_moddown_without_rescale_fp64_against_integer(lib, N, L, K, batch):
+    """Key-switch without a rescale: the FP64 ModDown + pass-through kernel (ks.mdr_fp64 = 1), with the
+    output limbs in one slice (it clears the divided rows) and in several, against the sequential
+    integer division and add (0), every allocated row compared; the first job against the oracle."""
+    s = Setup(N, L, K, 900 + N + K)
+    key = s.key(L, 1)
+    ksk = s.outer([key, None])
+    ins = [s.ct(2, s.lvl_mask) for _ in range(batch)]
+    got, saved = {}, lib.vfhe_hip_get_option(b"ks.mdr_fp64")
+    try:
+        for fp in (1, 0):
+            assert lib.vfhe_hip_set_option(b"ks.mdr_fp64", fp) == 0
+            outs = [s.pool.sample(1, s.ext_mask) for _ in ins]
+            n0 = lib.vfhe_hip_get_option(b"stat.mdr_fp64_launches")
+            lib.vfhe_hip_mlwe_keyswitch_batch(_native.voidp_array(outs), _native.voidp_array([c for _, c in ins]),
+                                              batch, ksk)
+            assert (lib.vfhe_hip_get_option(b"stat.mdr_fp64_launches") > n0) == bool(fp)
+            got[fp] = [s.pool.read_sample(o) for o in outs]
+            assert s.pool.sample_masks(outs[-1]) == [s.lvl_mask] * 2
+    finally:
+        lib.vfhe_hip_set_option(b"ks.mdr_fp64", saved)
+    for a, b in zip(got[1], got[0]):
+        assert np.array_equal(a, b)
+    ref = np.zeros((2, L + K, N), dtype=np.uint64)
+    mref = s.octx.ghs_keyswitch(ref, 1, ins[0][0], 2, s.lvl_mask, [key[0], None], s.ext_mask)
+    s.check(got[1][0], ref, mref)
+
+
 @pytest.mark.parametrize("rescale", [False, True])
 def test_multiply_pass_through_folded_into_key_mac(lib, rescale):
     """ks.fold = 1: the tensor's linear and constant slots stay in NTT form and enter the fused

@@ -1713,7 +1713,7 @@ static const void *div_consts(incNTT t, uint64_t mask, uint64_t chunk, const std
     return d_consts;
 }
 
-// Constant rows of k_moddown_rescale_fp for the limbs of `mask`, dividing by the special
+// Constant rows of k_moddown_fp (resc = -1: no rescale) for the limbs of `mask`, dividing by the special
 // primes dv (ascending, the limbs of `down`) and then by limb `resc`: the sequential round
 // divisions (rns_polynomial.c:939-976) written as one affine map per limb.  With
 // inv_j(q) = p_j^-1 mod q and h_j(q) = floor(p_j/2) mod q:
@@ -1748,7 +1748,7 @@ static const void *mdr_fp_consts(incNTT t, uint64_t mask, uint64_t down, const s
         put((size_t)k * W, G, pk);
         cs[(size_t)k * W + 1] = make_double2(centred(c, pk), 0.0);
     }
-    const uint64_t qr = t->ntt[resc]->q;
+    const uint64_t qr = resc >= 0 ? t->ntt[resc]->q : 0;
     for (uint64_t i = 0; i < l; i++) {
         if (!ACTIVE(mask, i) || ACTIVE(down, i)) continue;
         const uint64_t qi = t->ntt[i]->q;
@@ -1757,9 +1757,9 @@ static const void *mdr_fp_consts(incNTT t, uint64_t mask, uint64_t down, const s
         uint64_t hs = 0;
         for (int k = 0; k < K; k++) hs = (hs + mulmod_h((t->ntt[dv[k]]->q / 2) % qi, Gk[k], qi)) % qi;
         const size_t row = (size_t)(4 + i) * W;
-        if ((int)i == resc) {
+        if (resc < 0 || (int)i == resc) {
             put(row, Gk[0], qi);
-            cs[row + 2] = make_double2(centred((hs + qr / 2) % qi, qi), 0.0);
+            cs[row + 2] = make_double2(centred((hs + qr / 2) % qi, qi), 0.0);   // qr = 0 without a rescale
             for (int k = 0; k < K; k++) put(row + 4 + k, neg(Gk[k], qi), qi);
         } else {
             const uint64_t A = inverse_mod(qr % qi, qi);
@@ -1992,24 +1992,45 @@ extern "C" void polynomial_RNSc_scaled_lift(RNSc_Polynomial out, RNSc_Polynomial
 // ---------------------------------------------------------------------------
 // Automorphism (rns_polynomial.c:996-1035)
 // ---------------------------------------------------------------------------
+// Rows of the automorphism X -> X^gen, launched together: an odd gen is read in output order with
+// gen^-1 mod 2N, an even one (no bijection) is written coefficient by coefficient.
+struct vh_permute_rows {
+    std::vector<vh_item> odd, even;
+    void add(RNS_Polynomial out, RNS_Polynomial in, uint64_t gen)
+    {
+        const uint64_t N = out->ntt->N;
+        VH_REQUIRE(out != in && gen > 0 && gen < 2 * N);
+        dev_ready(in); dev_ready(out);
+        out->rns_mask = in->rns_mask;
+        uint64_t inv = gen;   // Newton: doubles the correct low bits, 3 to start with
+        for (int k = 0; k < 5; k++) inv *= 2 - gen * inv;
+        for_active(out->rns_mask, std::min(out->ntt->l, out->allocated_l), [&](uint64_t j) {
+            (gen & 1 ? odd : even).push_back(mk_item(drow(in, j), drow(out, j), (uint32_t)j, nullptr, out->ntt->split_degree, 0,
+                                                     (uint32_t)(gen & 1 ? inv & (2 * N - 1) : gen)));
+        });
+    }
+    void run(incNTT t)
+    {
+        for (auto *v : {&odd, &even})
+            for (size_t off = 0; off < v->size(); off += VH_MAX_GRID_Y) {
+                const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, v->size() - off);
+                std::vector<vh_item> chunk(v->begin() + off, v->begin() + off + cnt);
+                vh_prof_scope ps_(VH_PROF_OTHER);
+                if (v == &odd) VH_LAUNCH(vh_launch_permute_odd(S(), vh_stage_vec(chunk), cnt, VPOOL(t)->d_limbs, t->N));
+                else VH_LAUNCH(vh_launch_permute(S(), vh_stage_vec(chunk), cnt, VPOOL(t)->d_limbs, t->N));
+            }
+    }
+};
+
 static void permute_into(RNS_Polynomial out, RNS_Polynomial in, uint64_t gen)
 {
-    VH_REQUIRE(out != in && gen > 0 && gen < 2 * out->ntt->N);
-    dev_ready(in); dev_ready(out);
-    out->rns_mask = in->rns_mask;
-    std::vector<vh_item> perm, zero;
+    vh_permute_rows rows;
+    rows.add(out, in, gen);
+    rows.run(out->ntt);
     const uint64_t l = std::min(out->ntt->l, out->allocated_l);
-    for (uint64_t j = 0; j < l; j++) {
-        if (ACTIVE(out->rns_mask, j))
-            perm.push_back(mk_item(drow(in, j), drow(out, j), (uint32_t)j, nullptr, out->ntt->split_degree, 0, (uint32_t)gen));
-        else
-            zero.push_back(mk_item(nullptr, drow(out, j), (uint32_t)j));
-    }
-    if (!perm.empty())
-        {
-            vh_prof_scope ps_(VH_PROF_OTHER);
-            VH_LAUNCH(vh_launch_permute(S(), vh_stage_vec(perm), (unsigned)perm.size(), DL(out), out->ntt->N));
-        }
+    std::vector<vh_item> zero;
+    for (uint64_t j = 0; j < l; j++)
+        if (!ACTIVE(out->rns_mask, j)) zero.push_back(mk_item(nullptr, drow(out, j), (uint32_t)j));
     run_eltwise(zero, DL(out), VH_OP_ZERO, out->ntt->N);
 }
 
@@ -2542,6 +2563,15 @@ static void gadget_batch(const std::vector<RNS_MLWE> &outs, const std::vector<st
 
 }
 
+// Slices of k_moddown_fp over the output limbs: a launch below two workgroups per CU spreads them,
+// at least two limbs each, towards four workgroups per CU; a fuller one keeps a single slice, which
+// reads the special rows once and clears them in the same pass.
+static unsigned moddown_slices(uint64_t jobs, uint64_t nout, uint64_t N)
+{
+    const uint64_t wgs = jobs * ((N + 511) / 512), cus = (uint64_t)C.cus;
+    return wgs >= 2 * cus ? 1 : (unsigned)std::max<uint64_t>(1, std::min(nout / 2, (4 * cus + wgs - 1) / wgs));
+}
+
 // mlwe_RNSc_GHS_hybrid_keyswitch (mlwe.c:557-598) for a batch whose jobs may
 // differ in level (masks) and key: job i switches ins[i] with ksks[i].  All jobs
 // share the ring and the output rank.
@@ -2597,17 +2627,27 @@ static void keyswitch_batch(const std::vector<RNS_MLWE> &outs, const std::vector
         }
     ntt_rows(pairs, 1);
 
-    // Jobs finished in one pass: a one-prime rescale, at most VH_MAX_DIV special primes,
-    // one mask for every output component, pass-through inputs covering it.
+    // Jobs finished in one pass: at most VH_MAX_DIV special primes, one mask for every output
+    // component, pass-through inputs covering it, and a one-prime rescale or (FP64 limbs, at most 4
+    // special primes) none.  Jobs of one mask, special primes and rescale share a launch.
+    incNTT t = outs[0]->b->ntt;
+    auto fp_ok = [&](uint64_t m, uint64_t down) {
+        bool fp = OPT.mdr_fp64 && __builtin_popcountll(down) <= 4;
+        for_active(m, l, [&](uint64_t i) { fp = fp && P->h_limbs[i].fp64; });
+        return fp;
+    };
     std::vector<char> fused(B, 0);
-    for (size_t bi = 0; bi < B && !rescale.empty(); bi++) {
+    std::map<std::tuple<uint64_t, uint64_t, uint64_t>, std::vector<size_t>> groups;   // (mask, special, rescale)
+    for (size_t bi = 0; bi < B; bi++) {
         const auto oc = comps(outs[bi]);
         const uint64_t m = oc[0]->rns_mask, down = m & ~ins[bi]->b->rns_mask, keep = m & ~down;
-        bool ok = __builtin_popcountll(rescale[bi]) == 1 && (rescale[bi] & keep) && down &&
-                  __builtin_popcountll(down) <= VH_MAX_DIV;
+        const uint64_t resc = rescale.empty() ? 0 : rescale[bi];
+        bool ok = down && __builtin_popcountll(down) <= VH_MAX_DIV &&
+                  (resc ? __builtin_popcountll(resc) == 1 && (resc & keep) : fp_ok(m, down));
         for (size_t c = 0; c < oc.size() && ok; c++)
             ok = oc[c]->rns_mask == m && (!pass[bi][c] || (pass[bi][c]->rns_mask & keep) == keep);
         fused[bi] = ok;
+        if (ok) groups[std::make_tuple(m, down, resc)].push_back(bi);
     }
     for (auto &g : by_divide) {
         std::vector<RNS_Polynomial> rest;
@@ -2620,36 +2660,9 @@ static void keyswitch_batch(const std::vector<RNS_MLWE> &outs, const std::vector
         if (g.first) run_division(rest, g.first, true);
     }
     std::vector<vh_item> adds;
-    std::vector<vh_mdr_job> mdr;
-    std::vector<vh_item> zero;
-    uint64_t mdr_mask = 0, mdr_down = 0, mdr_resc = 0;
     for (size_t bi = 0; bi < B; bi++) {
+        if (fused[bi]) continue;
         const auto oc = comps(outs[bi]);
-        if (fused[bi]) {
-            const uint64_t m = oc[0]->rns_mask, down = m & ~ins[bi]->b->rns_mask, keep = m & ~down;
-            if (mdr.empty()) { mdr_mask = m; mdr_down = down; mdr_resc = rescale[bi]; }
-            if (m != mdr_mask || down != mdr_down || rescale[bi] != mdr_resc) { fused[bi] = 0; }
-            else {
-                for (size_t c = 0; c < oc.size(); c++) {
-                    vh_mdr_job jb;
-                    memset(&jb, 0, sizeof(jb));
-                    jb.base = VP(oc[c])->d;
-                    jb.add = pass[bi][c] ? VP(pass[bi][c])->d : nullptr;
-                    jb.stride = N;
-                    jb.nl = (int)l;
-                    for (uint64_t i = 0; i < l; i++) if (ACTIVE(down, i)) jb.div_limb[jb.K++] = (int)i;
-                    jb.resc = __builtin_ctzll(rescale[bi]);
-                    for (uint64_t i = 0; i < l; i++)
-                        if (ACTIVE(keep, i) && !ACTIVE(rescale[bi], i)) jb.out_limb[jb.nout++] = (int)i;
-                    mdr.push_back(jb);
-                    for_active(down | rescale[bi], l, [&](uint64_t i) { zero.push_back(mk_item(nullptr, drow(oc[c], i), (uint32_t)i)); });
-                    oc[c]->rns_mask = keep & ~rescale[bi];
-                }
-                continue;
-            }
-            // a job of another mask or prime set: the sequential path (rare)
-            run_division(oc, down, true);
-        }
         for (size_t c = 0; c < oc.size(); c++) {
             RNS_Polynomial o = oc[c], x = pass[bi][c];
             if (!x) continue;
@@ -2659,26 +2672,50 @@ static void keyswitch_batch(const std::vector<RNS_MLWE> &outs, const std::vector
         }
     }
     run_eltwise(adds, P->d_limbs, VH_OP_ADD, N);
-    if (!mdr.empty()) {
-        std::vector<int> dv, rv = {__builtin_ctzll(mdr_resc)};
-        for (uint64_t i = 0; i < l; i++) if (ACTIVE(mdr_down, i)) dv.push_back((int)i);
-        incNTT t = outs[0]->b->ntt;
-        bool fp = OPT.mdr_fp64 && dv.size() <= 4;
-        for_active(mdr_mask, l, [&](uint64_t i) { fp = fp && P->h_limbs[i].fp64; });
-        const void *cd = fp ? nullptr : div_consts(t, mdr_mask, mdr_down, dv, true);
-        const void *cr = fp ? nullptr : div_consts(t, mdr_mask & ~mdr_down, mdr_resc, rv, true);
-        const void *cf = fp ? mdr_fp_consts(t, mdr_mask, mdr_down, dv, rv[0]) : nullptr;
+    for (auto &g : groups) {
+        const uint64_t m = std::get<0>(g.first), down = std::get<1>(g.first), resc = std::get<2>(g.first);
+        const uint64_t keep = m & ~down;
+        const int rl = resc ? __builtin_ctzll(resc) : -1;
+        std::vector<int> dv;
+        for (uint64_t i = 0; i < l; i++) if (ACTIVE(down, i)) dv.push_back((int)i);
+        std::vector<vh_mdr_job> mdr;
+        std::vector<vh_item> zero;
+        for (size_t bi : g.second) {
+            const auto oc = comps(outs[bi]);
+            for (size_t c = 0; c < oc.size(); c++) {
+                vh_mdr_job jb;
+                memset(&jb, 0, sizeof(jb));
+                jb.base = VP(oc[c])->d;
+                jb.add = pass[bi][c] ? VP(pass[bi][c])->d : nullptr;
+                jb.stride = N;
+                jb.nl = (int)l;
+                for (int d : dv) jb.div_limb[jb.K++] = d;
+                jb.resc = rl;
+                for (uint64_t i = 0; i < l; i++)
+                    if (ACTIVE(keep, i) && !ACTIVE(resc, i)) jb.out_limb[jb.nout++] = (int)i;
+                mdr.push_back(jb);
+                for_active(down | resc, l, [&](uint64_t i) { zero.push_back(mk_item(nullptr, drow(oc[c], i), (uint32_t)i)); });
+                oc[c]->rns_mask = keep & ~resc;
+            }
+        }
+        const bool fp = fp_ok(m, down);
+        const void *cd = fp ? nullptr : div_consts(t, m, down, dv, true);
+        const void *cr = fp ? nullptr : div_consts(t, keep, resc, {rl}, true);
+        const void *cf = fp ? mdr_fp_consts(t, m, down, dv, rl) : nullptr;
+        bool cleared = fp;
         for (size_t off = 0; off < mdr.size(); off += VH_MAX_GRID_Y) {
             const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, mdr.size() - off);
             std::vector<vh_mdr_job> chunk(mdr.begin() + off, mdr.begin() + off + cnt);
             vh_prof_scope ps_(VH_PROF_DIVISION);
             if (fp) {
-                VH_LAUNCH(vh_launch_moddown_rescale_fp(S(), vh_stage_vec(chunk), cnt, P->d_limbs, cf, N));
+                const unsigned slices = moddown_slices(cnt, (unsigned)mdr[0].nout, N);
+                VH_LAUNCH(vh_launch_moddown_fp(S(), vh_stage_vec(chunk), cnt, P->d_limbs, cf, N, resc != 0, slices));
                 g_mdr_fp64_launches++;
+                cleared = cleared && slices == 1;
             }
             else VH_LAUNCH(vh_launch_moddown_rescale(S(), vh_stage_vec(chunk), cnt, P->d_limbs, cd, cr, N, (int)dv.size()));
         }
-        run_eltwise(zero, P->d_limbs, VH_OP_ZERO, N);
+        if (!cleared) run_eltwise(zero, P->d_limbs, VH_OP_ZERO, N);
     }
     // jobs with a rescale not done above
     std::map<uint64_t, std::vector<RNS_Polynomial>> resc_groups;
@@ -2694,15 +2731,14 @@ extern "C" void mlwe_RNSc_GHS_hybrid_keyswitch(RNSc_MLWE out, RNSc_MLWE in, RNS_
     keyswitch_batch({out}, {in}, {ksk});
 }
 
+static void automorphism_batch(const std::vector<RNS_MLWE> &outs, const std::vector<RNS_MLWE> &ins,
+                               const std::vector<uint64_t> &gens, const std::vector<RNS_MLWE **> &ksks);
+
 extern "C" void mlwe_automorphism_RNSc_GHS(RNSc_MLWE out, RNSc_MLWE in, uint64_t gen, RNS_MLWE **ksk, uint64_t lvl)
 {
     (void)lvl;
     VH_ENTER;
-    RNSc_MLWE tmp = alloc_sample_raw(out->a[0]->ntt->N, out->r, out->a[0]->rns_mask, out->a[0]->ntt);
-    for (uint64_t i = 0; i < out->r; i++) permute_into(tmp->a[i], in->a[i], gen);
-    permute_into(tmp->b, in->b, gen);
-    keyswitch_batch({out}, {tmp}, {ksk});
-    free_mlwe_RNS_sample(tmp);
+    automorphism_batch({out}, {in}, {gen}, {ksk});
 }
 
 // mlwe_automorphism_RNSc_GHS (mlwe.c:314-326) for many inputs, each with its own
@@ -2713,13 +2749,15 @@ static void automorphism_batch(const std::vector<RNS_MLWE> &outs, const std::vec
     const size_t B = outs.size();
     VH_REQUIRE(B > 0 && ins.size() == B && gens.size() == B && ksks.size() == B);
     std::vector<RNS_MLWE> tmp(B);
+    vh_permute_rows rows;   // the temporaries' inactive rows are never read
     for (size_t bi = 0; bi < B; bi++) {
         RNS_MLWE o = outs[bi], x = ins[bi];
-        VH_REQUIRE(o != x && o->r == x->r);
+        VH_REQUIRE(o != x && o->r == x->r && o->a[0]->ntt == outs[0]->a[0]->ntt);
         tmp[bi] = alloc_sample_raw(o->a[0]->ntt->N, o->r, o->a[0]->rns_mask, o->a[0]->ntt);
-        for (uint64_t i = 0; i < o->r; i++) permute_into(tmp[bi]->a[i], x->a[i], gens[bi]);
-        permute_into(tmp[bi]->b, x->b, gens[bi]);
+        for (uint64_t i = 0; i < o->r; i++) rows.add(tmp[bi]->a[i], x->a[i], gens[bi]);
+        rows.add(tmp[bi]->b, x->b, gens[bi]);
     }
+    rows.run(outs[0]->a[0]->ntt);
     keyswitch_batch(outs, tmp, ksks);
     for (auto t : tmp) free_mlwe_RNS_sample(t);
 }

@@ -52,8 +52,8 @@ struct vh_div_job {
     int out_limb[VH_MAX_LIMBS];
 };
 
-// ModDown by K special primes, pass-through add and rescale by one prime of a
-// key-switch output component (k_moddown_rescale).
+// ModDown by K special primes, pass-through add and (resc >= 0) rescale by one prime of a
+// key-switch output component (k_moddown_rescale, k_moddown_fp).
 struct vh_mdr_job {
     uint64_t *base;          // device rows of the component, limb-major
     const uint64_t *add;     // rows of the pass-through polynomial (same layout), or null
@@ -61,7 +61,7 @@ struct vh_mdr_job {
     int K;                   // special primes
     int nl;                  // pool size (row count of the constant tables)
     int nout;                // output limbs (the rescale limb excluded)
-    int resc;                // the rescale limb
+    int resc;                // the rescale limb, or -1
     int div_limb[VH_MAX_DIV];
     int out_limb[VH_MAX_LIMBS];
 };
@@ -184,16 +184,18 @@ hipError_t vh_launch_split_mul(hipStream_t st, const vh_item *items, unsigned ni
 // cdown: K x nl division constants of the special primes; cresc: 1 x nl of the rescale prime.
 hipError_t vh_launch_moddown_rescale(hipStream_t st, const vh_mdr_job *jobs, unsigned njobs, const vh_limb *limbs,
                                      const void *cdown, const void *cresc, uint64_t n, int kmax);
-// FP64 form (every limb below 2^50, K <= 4): cs holds the constant rows built by the
+// FP64 form (every limb below 2^50, K <= 4), with or without the rescale: cs holds the constant rows built by the
 // engine (4 special rows, then one row per pool limb, VH_MDR_W double2 each).
 #define VH_MDR_W 8
-hipError_t vh_launch_moddown_rescale_fp(hipStream_t st, const vh_mdr_job *jobs, unsigned njobs, const vh_limb *limbs,
-                                        const void *cs, uint64_t n);
+hipError_t vh_launch_moddown_fp(hipStream_t st, const vh_mdr_job *jobs, unsigned njobs, const vh_limb *limbs,
+                                const void *cs, uint64_t n, int resc, unsigned slices);
 hipError_t vh_launch_division(hipStream_t st, const vh_div_job *jobs, unsigned njobs, unsigned nout,
                               const vh_limb *limbs, const void *consts, uint64_t n, int kmax);
 hipError_t vh_launch_base_conversion(hipStream_t st, const vh_bconv_job *jobs, unsigned njobs, unsigned nout,
                                      const vh_limb *limbs, const void *consts, uint64_t n);
 hipError_t vh_launch_permute(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, uint64_t N);
+// The same for odd gen, item.aux = gen^-1 mod 2N.
+hipError_t vh_launch_permute_odd(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, uint64_t N);
 // Forward row pass (last 8 stages) of every digit fused with the inner product
 // out_c = -sum_d digit_d * key[d][c]; modup holds the column-pass output.
 // FP64 path, 13 <= logn <= 16, comps 1 or 2.

@@ -1220,79 +1220,6 @@ k_moddown_rescale(const vh_mdr_job *__restrict__ jobs, const vh_limb *__restrict
     }
 }
 
-// The same ModDown + pass-through + rescale on the FP64 path (every limb below 2^50,
-// at most 4 special primes).  The K sequential round divisions of the reference
-// (rns_polynomial.c:939-976, ascending special primes, then the rescale prime) are
-// affine in the row values and in the carried t_k = (special row k after the
-// divisions before it + floor(p_k/2)) mod p_k, so with the products of inverses
-// folded into per-limb constants (built on the host, exact):
-//   t_k   = canon(v_k * G_k + c_k + sum_{j<k} t_j * g_kj)                 mod p_k
-//   t_r   = canon(x_r * X_r + add_r + C_r + sum_k t_k * T_rk)             mod q_r
-//   out_i = canon(x_i * X_i + add_i * A_i + C_i + t_r * R_i + sum_k t_k * T_ik)  mod q_i
-// Each product is vh_mulmod_tw against a centred constant ({w, RN(w/q)}): |term| <= 3q/4,
-// so with K <= 4 every sum stays below 6q < 2^53 and the result is the reference's,
-// bit for bit.  Constant rows (stride VH_MDR_W double2): rows 0..3 the special primes
-// [G, c, g_k0..g_k3], then row 4 + limb for every limb of the pool [X, A, C, R, T_0..T_3]
-// (C in .x only).
-__global__ void __launch_bounds__(256)
-k_moddown_rescale_fp(const vh_mdr_job *__restrict__ jobs, const vh_limb *__restrict__ limbs,
-                     const double2 *__restrict__ cs, uint64_t n)
-{
-    constexpr int KMAX = 4, W = VH_MDR_W;
-    const vh_mdr_job &jb = jobs[blockIdx.y];
-    const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= n) return;
-    const int K = jb.K;
-    const VH_GLOBAL uint64_t *base = vh_global(jb.base);
-    const VH_GLOBAL uint64_t *add = jb.add ? vh_global(jb.add) : nullptr;
-    auto row = [&](const VH_GLOBAL uint64_t *b, int limb) -> double { return vh_u2d(b[(uint64_t)limb * jb.stride + x]); };
-    double t[KMAX];
-#pragma unroll
-    for (int k = 0; k < KMAX; k++) {
-        if (k >= K) continue;   // (continue, not break: the loop unrolls fully)
-        const int lk = jb.div_limb[k];
-        const vh_limb &L = limbs[lk];
-        const double2 *c = cs + k * W;
-        double s = c[1].x + vh_mulmod_tw(row(base, lk), c[0].x, c[0].y, L.qd);
-#pragma unroll
-        for (int j = 0; j < KMAX; j++)
-            if (j < k) s += vh_mulmod_tw(t[j], c[2 + j].x, c[2 + j].y, L.qd);
-        t[k] = vh_canon(s, L.qd, L.qinv);
-    }
-    const int lr = jb.resc;
-    double tr;
-    {
-        const vh_limb &L = limbs[lr];
-        const double2 *c = cs + (KMAX + lr) * W;
-        double s = c[2].x + vh_mulmod_tw(row(base, lr), c[0].x, c[0].y, L.qd);
-        if (add) s += row(add, lr);
-#pragma unroll
-        for (int k = 0; k < KMAX; k++)
-            if (k < K) s += vh_mulmod_tw(t[k], c[4 + k].x, c[4 + k].y, L.qd);
-        tr = vh_canon(s, L.qd, L.qinv);
-    }
-    VH_GLOBAL uint64_t *outb = vh_global(jb.base);
-    for (int o = 0; o < jb.nout; o++) {
-        const int li = jb.out_limb[o];
-        const vh_limb &L = limbs[li];
-        const double2 *c = cs + (KMAX + li) * W;
-        double s = c[2].x + vh_mulmod_tw(row(base, li), c[0].x, c[0].y, L.qd) + vh_mulmod_tw(tr, c[3].x, c[3].y, L.qd);
-        if (add) s += vh_mulmod_tw(row(add, li), c[1].x, c[1].y, L.qd);
-#pragma unroll
-        for (int k = 0; k < KMAX; k++)
-            if (k < K) s += vh_mulmod_tw(t[k], c[4 + k].x, c[4 + k].y, L.qd);
-        outb[(uint64_t)li * jb.stride + x] = vh_d2u(vh_canon(s, L.qd, L.qinv));
-    }
-}
-
-hipError_t vh_launch_moddown_rescale_fp(hipStream_t st, const vh_mdr_job *jobs, unsigned njobs, const vh_limb *limbs,
-                                        const void *cs, uint64_t n)
-{
-    const dim3 grid((unsigned)((n + 255) / 256), njobs);
-    VH_KL(k_moddown_rescale_fp, grid, dim3(256), 0, st, jobs, limbs, (const double2 *)cs, n);
-    return hipGetLastError();
-}
-
 hipError_t vh_launch_moddown_rescale(hipStream_t st, const vh_mdr_job *jobs, unsigned njobs, const vh_limb *limbs,
                                      const void *cdown, const void *cresc, uint64_t n, int kmax)
 {
@@ -1355,6 +1282,45 @@ k_permute(const vh_item *__restrict__ items, const vh_limb *__restrict__ limbs, 
         if (idx & N) v = (int64_t)((uint64_t)0 - (uint64_t)v);
         uint64_t a = vh_reduce64(v < 0 ? (uint64_t)0 - (uint64_t)v : (uint64_t)v, L.q, L.mu64);
         it.dst[dst] = (v < 0 && a) ? L.q - a : a;
+    }
+}
+
+// The same for an odd gen (a bijection) read in output order: coefficient X^d takes coefficient i =
+// d gen^-1 mod 2N, negated when i >= N.  items: aux = gen^-1 mod 2N, scalar = S.  Bound by the
+// scattered side, one 128-byte line per element, which has to stay in one L2: consecutive workgroups
+// go to the 8 XCDs in turn, so workgroup b takes row (b mod 8) + 8 (b / 8 / tiles) -- all of a row on one
+// XCD -- and streams its coalesced writes past the caches.
+__global__ void __launch_bounds__(256)
+k_permute_odd(const vh_item *__restrict__ items, unsigned nitems, const vh_limb *__restrict__ limbs, uint32_t N,
+              unsigned tiles)
+{
+    const unsigned lane8 = blockIdx.x & 7, grp = blockIdx.x >> 3;
+    const unsigned row = lane8 + 8 * (grp / tiles), tile = grp % tiles;
+    if (row >= nitems) return;
+    const vh_item &it = items[row];
+    const vh_limb &L = limbs[it.limb];
+    const uint64_t q = L.q, mu = L.mu64;
+    const uint32_t S = (uint32_t)it.scalar, slog = 31 - __builtin_clz(S), n = N >> slog, nlog = 31 - __builtin_clz(n);
+    const VH_GLOBAL uint64_t *src = vh_global(it.src);
+    VH_GLOBAL uint64_t *dst = vh_global(it.dst);
+    const uint32_t e0 = tile * 1024 + threadIdx.x;
+    int64_t v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const uint32_t e = e0 + 256 * k;
+        v[k] = 0;
+        if (e >= N) continue;
+        const uint32_t d = (e >> nlog) + ((e & (n - 1)) << slog);
+        const uint32_t i = (d * it.aux) & (2 * N - 1);
+        v[k] = (int64_t)src[((i & (S - 1)) << nlog) + ((i & (N - 1)) >> slog)];
+        if (i & N) v[k] = (int64_t)((uint64_t)0 - (uint64_t)v[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const uint32_t e = e0 + 256 * k;
+        if (e >= N) continue;
+        const uint64_t a = vh_reduce64(v[k] < 0 ? (uint64_t)0 - (uint64_t)v[k] : (uint64_t)v[k], q, mu);
+        vh_st(dst + e, (v[k] < 0 && a) ? q - a : a);
     }
 }
 
@@ -1640,6 +1606,14 @@ hipError_t vh_launch_base_conversion(hipStream_t st, const vh_bconv_job *jobs, u
 hipError_t vh_launch_permute(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, uint64_t N)
 {
     VH_KL(k_permute, dim3(vh_blocks(N, 256, 64), nitems), dim3(256), 0, st, items, limbs, N);
+    return hipGetLastError();
+}
+
+hipError_t vh_launch_permute_odd(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, uint64_t N)
+{
+    if (N < 2 || N > (1u << 30) || nitems == 0) return hipErrorInvalidValue;
+    const unsigned tiles = (unsigned)((N + 1023) / 1024);
+    VH_KL(k_permute_odd, dim3(8 * tiles * ((nitems + 7) / 8)), dim3(256), 0, st, items, nitems, limbs, (uint32_t)N, tiles);
     return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
-// vh_keyswitch.hip -- key-switch inner product fused into the forward row pass of the
-// ModUp digits (FP64 path, N = 2^13 .. 2^16, at most two output components).
+// vh_keyswitch.hip -- key-switch kernels of the FP64 path: the inner product fused into the forward row
+// pass of the ModUp digits (N = 2^13 .. 2^16, at most two output components), and the ModDown.
 #include "vh_device.h"
 #include "vh_kernels.h"
 
@@ -206,5 +206,116 @@ hipError_t vh_launch_row_mac(hipStream_t st, const vh_mac_job *jobs, unsigned nj
     const int xcd = (grid.y * grid.z) % 8 == 0;
     if (comps == 1) VH_KL(k_row_mac<1>, grid, dim3(256), 0, st, jobs, limbs, kptr, logn, xcd);
     else VH_KL(k_row_mac<2>, grid, dim3(256), 0, st, jobs, limbs, kptr, logn, xcd);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// ModDown of a key-switch output component, with the pass-through add, and with RESC the CKKS
+// rescale that follows, on the FP64 path (every limb below 2^50, at most 4 special primes).  The K
+// sequential round divisions of the reference (rns_polynomial.c:939-976, ascending special primes,
+// then the rescale prime) are affine in the row values and in the carried t_k = (special row k after
+// the divisions before it + floor(p_k/2)) mod p_k, so with the products of inverses folded into
+// per-limb constants (built on the host, exact):
+//   t_k   = canon(v_k G_k + c_k + sum_{j<k} t_j g_kj)                                mod p_k
+//   t_r   = canon(x_r X_r + add_r + C_r + sum_k t_k T_rk)                            mod q_r
+//   out_i = canon(x_i X_i + add_i A_i + C_i + t_r R_i + sum_k t_k T_ik)              mod q_i
+// and without the rescale  out_i = canon(x_i X_i + C_i + sum_k t_k T_ik) + add_i.
+// Each product is vh_mulmod_tw against a centred constant ({w, RN(w/q)}): |term| <= 3q/4, so with
+// K <= 4 every sum stays below 6q < 2^53 and the result is the reference's, bit for bit.  Constant
+// rows (stride VH_MDR_W double2): rows 0..3 the special primes [G, c, g_k0..g_k3], then row 4 +
+// limb for every limb of the pool [X, A, C, R, T_0..T_3] (C in .x only).
+//
+// A thread owns two adjacent coefficients (16-byte accesses).  Bound by HBM at large batches.  A launch of
+// few workgroups runs its output limbs one after another and waits for memory at each, so the
+// limbs are then divided over gridDim.z slices, each forming the chain t again (64 workgroups for one
+// multiply at N = 2^14, 11 + 4 limbs: 16 us in one slice).  With one slice the divided rows are cleared
+// here; with more, another slice may still read them and the caller clears them.
+// ---------------------------------------------------------------------------
+template <bool RESC>
+__global__ void __launch_bounds__(256)
+k_moddown_fp(const vh_mdr_job *__restrict__ jobs, const vh_limb *__restrict__ limbs, const double2 *__restrict__ cs,
+             unsigned n)
+{
+    constexpr int KMAX = 4, W = VH_MDR_W;
+    const vh_mdr_job &jb = jobs[blockIdx.y];
+    const unsigned x = (blockIdx.x * 256 + threadIdx.x) * 2;
+    if (x >= n) return;
+    const int K = jb.K;
+    VH_GLOBAL uint64_t *base = vh_global(jb.base);
+    const VH_GLOBAL uint64_t *add = jb.add ? vh_global(jb.add) : nullptr;
+    auto at = [&](int limb) -> size_t { return (size_t)limb * jb.stride + x; };
+    double t[KMAX][2];
+#pragma unroll
+    for (int k = 0; k < KMAX; k++) {
+        if (k >= K) continue;   // (continue, not break: the loop unrolls fully)
+        const int lk = jb.div_limb[k];
+        const vh_limb &L = limbs[lk];
+        const double2 *c = cs + k * W;
+        uint64_t v[2];
+        vh_ld2(base + at(lk), v[0], v[1]);
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            double s = c[1].x + vh_mulmod_tw(vh_u2d(v[e]), c[0].x, c[0].y, L.qd);
+#pragma unroll
+            for (int j = 0; j < KMAX; j++)
+                if (j < k) s += vh_mulmod_tw(t[j][e], c[2 + j].x, c[2 + j].y, L.qd);
+            t[k][e] = vh_canon(s, L.qd, L.qinv);
+        }
+    }
+    double tr[2];
+    if (RESC) {
+        const int lr = jb.resc;
+        const vh_limb &L = limbs[lr];
+        const double2 *c = cs + (KMAX + lr) * W;
+        uint64_t v[2], a[2] = {0, 0};
+        vh_ld2(base + at(lr), v[0], v[1]);
+        if (add) vh_ld2(add + at(lr), a[0], a[1]);
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            double s = c[2].x + vh_mulmod_tw(vh_u2d(v[e]), c[0].x, c[0].y, L.qd) + vh_u2d(a[e]);
+#pragma unroll
+            for (int k = 0; k < KMAX; k++)
+                if (k < K) s += vh_mulmod_tw(t[k][e], c[4 + k].x, c[4 + k].y, L.qd);
+            tr[e] = vh_canon(s, L.qd, L.qinv);
+        }
+    }
+    const int per = (jb.nout + (int)gridDim.z - 1) / (int)gridDim.z;
+    const int o0 = (int)blockIdx.z * per, o1 = o0 + per < jb.nout ? o0 + per : jb.nout;
+    for (int o = o0; o < o1; o++) {
+        const int li = jb.out_limb[o];
+        const vh_limb &L = limbs[li];
+        const double2 *c = cs + (KMAX + li) * W;
+        uint64_t v[2], a[2] = {0, 0}, r[2];
+        vh_ld2(base + at(li), v[0], v[1]);
+        if (add) vh_ld2(add + at(li), a[0], a[1]);
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            double s = c[2].x + vh_mulmod_tw(vh_u2d(v[e]), c[0].x, c[0].y, L.qd);
+            if (RESC) {
+                s += vh_mulmod_tw(tr[e], c[3].x, c[3].y, L.qd);
+                if (add) s += vh_mulmod_tw(vh_u2d(a[e]), c[1].x, c[1].y, L.qd);
+            }
+#pragma unroll
+            for (int k = 0; k < KMAX; k++)
+                if (k < K) s += vh_mulmod_tw(t[k][e], c[4 + k].x, c[4 + k].y, L.qd);
+            r[e] = vh_d2u(vh_canon(s, L.qd, L.qinv));
+            if (!RESC && add) r[e] = vh_reduce64(r[e] + a[e], L.q, L.mu64);   // any 64-bit addend, as the elementwise add
+        }
+        vh_st2(base + at(li), r[0], r[1]);
+    }
+    if (gridDim.z == 1) {
+        for (int k = 0; k < K; k++) vh_st2(base + at(jb.div_limb[k]), 0, 0);
+        if (RESC) vh_st2(base + at(jb.resc), 0, 0);
+    }
+}
+
+// slices: output-limb slices (1: the kernel clears the divided rows).
+hipError_t vh_launch_moddown_fp(hipStream_t st, const vh_mdr_job *jobs, unsigned njobs, const vh_limb *limbs,
+                                const void *cs, uint64_t n, int resc, unsigned slices)
+{
+    if (n < 2 || n > (1u << 30) || (n & 1) || slices < 1) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((n + 511) / 512), njobs, slices);
+    if (resc) VH_KL(k_moddown_fp<true>, grid, dim3(256), 0, st, jobs, limbs, (const double2 *)cs, (unsigned)n);
+    else VH_KL(k_moddown_fp<false>, grid, dim3(256), 0, st, jobs, limbs, (const double2 *)cs, (unsigned)n);
     return hipGetLastError();
 }
