@@ -184,7 +184,7 @@ struct vh_opts {
     long ntt_col_wide = 1;    // pipelined column passes: 512-thread workgroups over 32-column tiles
     long ntt_tile_grid = 15;   // pipelined passes launched one tile per workgroup instead of
                               // persistent: bit 0 forward column, 1 forward row, 2 inverse row,
-                              // 3 inverse column, 4 the fused product's row kernel
+                              // 3 inverse column (bit 4 chooses nothing)
     long xcd_lag = 3;         // persistent mode: queue slots between an item's two passes
     long xcd_occ = 2;         // persistent mode: workgroups per CU (2 or 4)
     long xcd_l2 = 1;          // persistent mode: the first pass stores its intermediate with
@@ -3894,9 +3894,7 @@ static void fused_product_launches(std::vector<vh_item> &col, std::vector<vh_ite
             const unsigned nb3 = ((OPT.ntt_tile_grid >> 3) & 1) ? UINT_MAX : C.pipe_blocks;
             if (which == 0 && pipe) VH_LAUNCH(vh_launch_ntt16p(S(), d, cnt, P->d_limbs, 0, logn, 0, R1, 1, 1, 0, nb0, col_wide(cnt, logn)));
             else if (which == 0) VH_LAUNCH(vh_launch_ntt16(S(), d, cnt, P->d_limbs, 0, logn, 0, R1, 1, 1, 0));
-            else if (which == 1 && pipe)
-                VH_LAUNCH(vh_launch_ntt16p_row_mul(S(), d, cnt, P->d_limbs, logn, C.cus, (int)((OPT.ntt_tile_grid >> 4) & 1)));
-            else if (which == 1) VH_LAUNCH(vh_launch_ntt16_row_mul_inv(S(), d, cnt, P->d_limbs, logn));
+            else if (which == 1) VH_LAUNCH(vh_launch_row_mul(S(), d, cnt, P->d_limbs, logn));
             else if (pipe) VH_LAUNCH(vh_launch_ntt16p(S(), d, cnt, P->d_limbs, 1, logn, 0, R1, 1, 0, 1, nb3, col_wide(cnt, logn)));
             else VH_LAUNCH(vh_launch_ntt16(S(), d, cnt, P->d_limbs, 1, logn, 0, R1, 1, 0, 1));
         }
@@ -4548,10 +4546,9 @@ static long autotune_generic(long nc, const std::function<void(long)> &apply, co
     return best;
 }
 
-// The fused product's schedule: its row kernel launched one tile per workgroup or
-// persistent (ntt.tile_grid bit 4) x its column passes at 256 threads, 512 threads by the
-// occupancy rule, or 512 threads always (ntt.col_wide 0 / 1 / 2): 6 candidates, timed on
-// the caller's operands (z is overwritten).
+// The fused product's schedule: its column passes at 256 threads, 512 threads by the occupancy rule,
+// or 512 threads always (ntt.col_wide 0 / 1 / 2), each timed twice on the caller's operands (z is
+// overwritten): 6 candidates, of which those that differ in ntt.tile_grid bit 4 alone run alike.
 extern "C" long vfhe_hip_autotune_product(RNS_Polynomial *z, RNS_Polynomial *x, RNS_Polynomial *y, uint64_t count,
                                           int reps, double *us_out)
 {

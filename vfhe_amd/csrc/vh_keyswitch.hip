@@ -1,7 +1,7 @@
 // vh_keyswitch.hip -- key-switch kernels of the FP64 path: the inner product fused into the forward row
 // pass of the ModUp digits (N = 2^13 .. 2^16, at most two output components), and the ModDown.
-#include "vh_device.h"
 #include "vh_kernels.h"
+#include "vh_row8.h"
 
 // ---------------------------------------------------------------------------
 // The column pass has left the lifted digit rows, transformed over their first
@@ -10,25 +10,15 @@
 //     out_c = -+ sum_d NTT(digit_d) * key[d][c]      (the mul_subto of gadget.c:22-37)
 // in registers, so the transformed digits never return to memory.
 //
-// A row has 32 threads with 8 values each, in three register phases:
-//   1  stages 0..2   k = t + 32 m                    (256-byte runs of the digit row)
-//   2  stages 3..5   k = 32 (t >> 2) + 4 m + (t & 3)
-//   3  stages 6..7   k = 128 (m >> 2) + 4 t + (m & 3)
-// with two exchanges through LDS inside the wave (row slices of 36 doubles per 32: the
-// reads of phase 2 touch every bank once).  Phase 3 leaves four adjacent elements per
-// lane, so the key rows, the pass-through rows and the output move as 16-byte words of
-// one contiguous kilobyte per 32 lanes.  (16 values per thread ending in 16 contiguous
-// elements made every key load touch 64 separate 128-byte lines.)
-// The row's 255 twiddles do not depend on the digit: they are formed once per workgroup
-// (table head times row factor, centred, as in k_ntt16p) into LDS.
+// Rows run as in vh_row8.h.  Its last phase leaves four adjacent elements per lane, so the key rows,
+// the pass-through rows and the output move as 16-byte words of one contiguous kilobyte per 32
+// lanes.  (16 values per thread ending in 16 contiguous elements made every key load touch 64
+// separate 128-byte lines.)
 // 8 values and two accumulators per thread leave room to load a digit's key words and the
 // next digit before the butterflies within 128 VGPRs: four workgroups per CU.
 // Measured for 32 ciphertexts at N = 2^16, 24 + 4 limbs (11.7 GB to read and write, 2.2 ms of
 // FP64 issue): 5.54 ms with 16 values per thread and contiguous key reads, 4.75 ms with those
 // values regrouped before the key reads, 3.80 ms in this form (3.1 TB/s).
-// Bounds: every twiddle is paired with w * RN(1/q), so a multiplied operand must stay
-// below 4q (see k_ntt16p): inputs are centred, four stages add at most 4q with the
-// multiplied operand of the fourth below 3.5q, then every value is centred again.
 //
 // Grid: x = ciphertext, y = tile, z = extended limb.  A key block is (y, z).
 // Consecutive workgroups are dealt round-robin over the 8 XCDs, so with `xcd` set the
@@ -38,15 +28,13 @@
 // measured on launches of 60 to 300 workgroups and gained nothing: the digit loop keeps its loads
 // in flight, and the partials' traffic costs what the extra workgroups save.
 // ---------------------------------------------------------------------------
-constexpr int VH_RM_PITCH = 288;   // doubles of one row's exchange slice (256 + 4 per 32)
-
 template <int C>
 __global__ void __launch_bounds__(256, 4)
 k_row_mac(const vh_mac_job *__restrict__ jobs, const vh_limb *__restrict__ limbs,
           const uint64_t *const *__restrict__ kptr, int logn, int xcd)
 {
-    constexpr int ROWS = 8, S = 256, T = 32;
-    __shared__ double lds[ROWS * VH_RM_PITCH];
+    constexpr int ROWS = vh_row8::ROWS, S = vh_row8::S, T = vh_row8::T;
+    __shared__ double lds[ROWS * vh_row8::PITCH];
     __shared__ double tws[ROWS][S];
     unsigned bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
     if (xcd) {   // bijective when gridDim.y * gridDim.z is a multiple of 8 (checked at launch)
@@ -66,18 +54,9 @@ k_row_mac(const vh_mac_job *__restrict__ jobs, const vh_limb *__restrict__ limbs
     const size_t n = (size_t)1 << logn;
     const int tid = threadIdx.x, g = tid / T, t = tid % T;
     const size_t sub = (size_t)by * ROWS + g;
-    {   // the rows' twiddles: entry e of row r = head e times the row's factor of e's stage
-        const int e = tid, sp = e ? 31 - __builtin_clz(e) : 0;
-        const double h = vh_global(reinterpret_cast<const double *>(L.tw_fwd))[2 * e];
-        const VH_GLOBAL double *rf = vh_global(reinterpret_cast<const double *>(L.rowf_fwd)) + ((size_t)by * ROWS * 8 + sp) * 2;
-#pragma unroll
-        for (int r = 0; r < ROWS; r++)
-            tws[r][e] = vh_center(vh_mulmod_tw(h, rf[16 * r], rf[16 * r + 1], q), q, qinv);
-        __syncthreads();
-    }
-    double *xs = lds + g * VH_RM_PITCH;
-    const double *tw = tws[g];
-    const int ta = t >> 2, tb = t & 3;
+    vh_row8::fill(tws, L, [&](int r) { return by * ROWS + r; });
+    __syncthreads();
+    const vh_row8 row(L, lds, tws);
     const size_t rowoff = sub * S, x0 = rowoff + 4 * t;
     const VH_GLOBAL uint64_t *dig = vh_global(jb.modup + (size_t)ti * n + rowoff + t);
     const size_t dstep = (size_t)jb.next * n;
@@ -88,21 +67,15 @@ k_row_mac(const vh_mac_job *__restrict__ jobs, const vh_limb *__restrict__ limbs
     for (int c = 0; c < C; c++)
 #pragma unroll
         for (int m = 0; m < 8; m++) acc[c][m] = 0.0;
-    auto bf = [&](double &a, double &b, double w) {
-        const double x = vh_mulmod_tw(b, w, w * qinv, q);
-        b = a - x;
-        a = a + x;
-    };
-
     uint64_t raw[8];
     if (D > 0) {
 #pragma unroll
         for (int m = 0; m < 8; m++) raw[m] = vh_ld(dig + 32 * m);
     }
     for (int d = 0; d < D; d++, kp += C) {
-        double v[8];
+        double v[1][8];
 #pragma unroll
-        for (int m = 0; m < 8; m++) v[m] = __longlong_as_double((long long)raw[m]);
+        for (int m = 0; m < 8; m++) v[0][m] = __longlong_as_double((long long)raw[m]);
         // this digit's key words, then the next digit: both land during the butterflies
         uint64_t kw[C][8];
 #pragma unroll
@@ -116,48 +89,11 @@ k_row_mac(const vh_mac_job *__restrict__ jobs, const vh_limb *__restrict__ limbs
             for (int m = 0; m < 8; m++) raw[m] = vh_ld(dig + (size_t)(d + 1) * dstep + 32 * m);
         }
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int s = 0; s < 3; s++) {
-            const int hm = 4 >> s;
-#pragma unroll
-            for (int m = 0; m < 8; m++)
-                if (!(m & hm)) bf(v[m], v[m + hm], tw[(1 << s) + (m >> (3 - s))]);
-        }
-        vh_wave_sync();   // every read of the previous digit's exchange is done
-#pragma unroll
-        for (int m = 0; m < 8; m++) xs[t + 36 * m] = v[m];
-        vh_wave_sync();
-#pragma unroll
-        for (int m = 0; m < 8; m++) v[m] = xs[36 * ta + 4 * m + tb];
-#pragma unroll
-        for (int s = 3; s < 6; s++) {
-            const int hm = 4 >> (s - 3);
-#pragma unroll
-            for (int m = 0; m < 8; m++)
-                if (!(m & hm)) bf(v[m], v[m + hm], tw[(1 << s) + (ta << (s - 3)) + (m >> (6 - s))]);
-            if (s == 3) {
-#pragma unroll
-                for (int m = 0; m < 8; m++) v[m] = vh_center(v[m], q, qinv);
-            }
-        }
-        // a thread overwrites the slots it read itself
-#pragma unroll
-        for (int m = 0; m < 8; m++) xs[36 * ta + 4 * m + tb] = v[m];
-        vh_wave_sync();
-#pragma unroll
-        for (int m = 0; m < 8; m++) v[m] = xs[144 * (m >> 2) + 4 * t + 4 * (t >> 3) + (m & 3)];
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const double w6 = tw[64 + 32 * h + t];
-            bf(v[4 * h], v[4 * h + 2], w6);
-            bf(v[4 * h + 1], v[4 * h + 3], w6);
-            bf(v[4 * h], v[4 * h + 1], tw[128 + 64 * h + 2 * t]);
-            bf(v[4 * h + 2], v[4 * h + 3], tw[128 + 64 * h + 2 * t + 1]);
-        }
+        row.fwd(v);
         const bool fourth = (d & 3) == 3;
 #pragma unroll
         for (int m = 0; m < 8; m++) {
-            const double a = vh_center(v[m], q, qinv);          // |a| <= q/2 + 1
+            const double a = row.centre(v[0][m]);                  // |a| <= q/2 + 1
 #pragma unroll
             for (int c = 0; c < C; c++) {
                 const double k = vh_u2d(kw[c][m]);
