@@ -4609,20 +4609,14 @@ struct vfhe_torus_batch {
 };
 static double2 *g_torus_consts = nullptr;
 
-// The transform constants (twiddles and twist), from long double cos / sin rounded once.
+// The transforms' twiddles: zeta^e = e^(i pi e / 1024), e < 2048, from long double cos / sin rounded once.
 static const double2 *torus_consts()
 {
     if (g_torus_consts) return g_torus_consts;
-    std::vector<double2> h(576);
+    std::vector<double2> h(2048);
     const long double pi = 3.141592653589793238462643383279502884L;
-    auto root = [&](long double num, long double den) {
-        const long double a = pi * num / den;
-        return make_double2((double)cosl(a), (double)sinl(a));
-    };
-    for (int k = 0; k < 8; k++)   // zeta^r w^(r k): angle pi r / 1024 - 2 pi r k / 512
-        for (int r = 0; r < 64; r++) h[k * 64 + r] = root((long double)r - 4.0L * ((r * k) % 512), 1024);
-    for (int a = 0; a < 8; a++)
-        for (int s = 0; s < 8; s++) h[512 + a * 8 + s] = root(-2.0L * ((8 * a * s) % 512), 512);
+    for (int e = 0; e < 2048; e++)
+        h[e] = make_double2((double)cosl(pi * e / 1024), (double)sinl(pi * e / 1024));
     double2 *d = nullptr;
     VH_CHECK(hipMalloc(&d, h.size() * sizeof(double2)));
     VH_CHECK(hipMemcpy(d, h.data(), h.size() * sizeof(double2), hipMemcpyHostToDevice));

@@ -26,14 +26,19 @@
 //   layout B  lane = 8 k2 + j0, slot = j1      between the passes
 //   layout C  lane = 8 k2 + k1, slot = k0      forward output (digit-reversed order),
 //                                              the key's storage order, inverse input
-// pass 1: DFT-8 over j2, twiddle w^((8 j1 + j0) k2); pass 2: DFT-8 over j1, twiddle
-// w^(8 j0 k1); pass 3: DFT-8 over j0.  The two exchanges go through a private LDS
-// slice of the wave with row pitches chosen so that every access spreads evenly over
-// the banks (pitch 72 for the A<->B exchange, 65 for B<->C).
-// The twist zeta^j, j = 64 j2 + r, splits as zeta^r zeta^(64 j2): the slot factor
-// c_j2 = zeta^(64 j2) multiplies the inputs (uniform constants), and the lane factor
-// zeta^r commutes with the DFT-8 over j2 and joins pass 1's twiddle, which becomes
-// zeta^r w^(r k2) for every k2 (k2 = 0 included); the inverse mirrors both.
+// B<->C goes through a private LDS slice of the wave with a row pitch of 65, which spreads every
+// access evenly over the banks.  A<->B swaps slot bits with lane bits 5..3: in registers where
+// many waves share the LDS (64 instructions instead of 32 LDS accesses, 6.07 ms against
+// 6.22 ms for 1024 samples), through LDS at pitch 72 where one workgroup has the CU and the
+// chain of instructions counts (2.50 ms against 2.65 ms for 3 samples).
+// Forward pass i evaluates the 8-term polynomial of a lane's slots at y_i e^(-2 pi i k / 8), k = 0..7,
+//     y_1 = zeta^64   y_2 = zeta^(8 - 32 k2)   y_3 = zeta^(1 - 4 (k2 + 8 k1)),
+// which covers the DFT-8, the twiddles before it and the pass's share of the twist: three radix-2
+// stages by y^4, y^2 and y of 12 butterflies with 6 fused operations each, 72 per pass.  (Plain
+// DFT-8s have 56, with 116 more for separate twiddles and twist: 6.33 ms for 1024 samples, 2.61 ms
+// for 3, and an rms error of 3.6e-16 instead of 2.3e-16 of the values' size.)
+// The inverse: a plain DFT-8 over k0, passes over k1 and k2 at y = zeta^(32 j0) and
+// zeta^(4 (8 j1 + j0)) with the conjugate DFT, then the untwist by zeta^-j.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -43,7 +48,7 @@ namespace {
 
 constexpr int VT_N = 1024, VT_M = 512;
 constexpr int VT_P1 = 72, VT_P2 = 65;          // exchange row pitches (doubles)
-constexpr int VT_XS = 8 * VT_P1;               // doubles per exchange array (>= 8 * VT_P2)
+constexpr int VT_XS = 8 * VT_P2;               // doubles of an exchange array that only B<->C uses
 
 // S = -1: X_k = sum_j x_j e^(-2 pi i jk / 8); S = +1: the same with +i (no scaling).
 template <int S>
@@ -103,36 +108,72 @@ __device__ __forceinline__ void vt_cmul(double &r, double &i, double wr, double 
     r = t;
 }
 
-// Twiddle tables in LDS, filled once per workgroup: t1[k 64 + r] = zeta^r w^(r k)
-// (pass 1 with the lane's twist factor, lane r, k = 0..7), t2[(s-1) 8 + a] = w^(8 a s)
-// (pass 2, a = lane mod 8, s = 1..7).  Per lane the reads are consecutive 16-byte words
-// (t1) or broadcasts (t2).
-constexpr int VT_T1 = 8 * 64, VT_T2 = 7 * 8;
-
-__device__ __forceinline__ void vt_fill_tw(double2 *t1, double2 *t2, const double2 *consts, int tid, int nthreads)
-{
-    for (int e = tid; e < VT_T1 + VT_T2; e += nthreads) {
-        if (e < VT_T1) {
-            t1[e] = consts[e];
-        } else {
-            const int s = (e - VT_T1) / 8 + 1, a = (e - VT_T1) % 8;
-            t2[e - VT_T1] = consts[512 + a * 8 + s];
-        }
+// A pass's twiddles: y^4, y^2, y and y e^(S 2 pi i / 8) for y = zeta^e, from the table of zeta's powers.
+struct vt_roots {
+    double2 w4, w2, w1, w3;
+    template <int S>
+    static __device__ __forceinline__ vt_roots at(const double2 *zeta, int e)
+    {
+        auto p = [&](int x) { return zeta[x & (2 * VT_N - 1)]; };
+        return {p(4 * e), p(2 * e), p(e), p(e + S * (VT_N / 4))};
     }
+};
+
+// (a, b) <- (a + w b, a - w b)
+__device__ __forceinline__ void vt_bf(double &ar, double &ai, double &br, double &bi, double wr, double wi)
+{
+    const double xr = __fma_rn(wr, br, __fma_rn(-wi, bi, ar)), xi = __fma_rn(wr, bi, __fma_rn(wi, br, ai));
+    br = __fma_rn(2.0, ar, -xr);
+    bi = __fma_rn(2.0, ai, -xi);
+    ar = xr;
+    ai = xi;
 }
 
-// Pass 2's twiddles w^(8 a s) of a = lane mod 8: read from the LDS table, or kept in registers.
-struct vt_t2_lds {
-    const double2 *t;
-    __device__ __forceinline__ double2 operator()(int s, int a) const { return t[(s - 1) * 8 + a]; }
-};
-struct vt_t2_reg {
-    double2 t[8];
-    __device__ __forceinline__ double2 operator()(int s, int) const { return t[s]; }
+// slot k <- sum_j (slot j) (y e^(S 2 pi i k / 8))^j
+template <int S>
+__device__ __forceinline__ void vt_pass(double *re, double *im, const vt_roots &t)
+{
+#pragma unroll
+    for (int j = 0; j < 4; j++) vt_bf(re[j], im[j], re[j + 4], im[j + 4], t.w4.x, t.w4.y);
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        vt_bf(re[j], im[j], re[j + 2], im[j + 2], t.w2.x, t.w2.y);
+        vt_bf(re[4 + j], im[4 + j], re[6 + j], im[6 + j], -S * t.w2.y, S * t.w2.x);   // times S i
+    }
+    vt_bf(re[0], im[0], re[1], im[1], t.w1.x, t.w1.y);                 // k = 0, 4
+    vt_bf(re[2], im[2], re[3], im[3], -S * t.w1.y, S * t.w1.x);        // k = 2, 6
+    vt_bf(re[4], im[4], re[5], im[5], t.w3.x, t.w3.y);                 // k = 1, 5
+    vt_bf(re[6], im[6], re[7], im[7], -S * t.w3.y, S * t.w3.x);        // k = 3, 7
+    auto order = [](double *v) {
+        const double v1 = v[1], v3 = v[3], v4 = v[4], v5 = v[5], v6 = v[6];
+        v[4] = v1; v[6] = v3; v[1] = v4; v[3] = v6; v[5] = v5;
+    };
+    order(re);
+    order(im);
+}
+
+// The inverse's twiddles in LDS: pass 2 by lane mod 8, pass 3 and the untwist by lane.
+struct vt_inv_tw {
+    double2 y2[4][8], y3[4][64], untwist[8][64];
+    __device__ __forceinline__ void fill(const double2 *zeta, int tid, int nthreads)
+    {
+        for (int l = tid; l < 64; l += nthreads) {
+            const vt_roots r = vt_roots::at<1>(zeta, 4 * l);
+            y3[0][l] = r.w4; y3[1][l] = r.w2; y3[2][l] = r.w1; y3[3][l] = r.w3;
+            if (l < 8) {
+                const vt_roots u = vt_roots::at<1>(zeta, 32 * l);
+                y2[0][l] = u.w4; y2[1][l] = u.w2; y2[2][l] = u.w1; y2[3][l] = u.w3;
+            }
+        }
+        for (int e = tid; e < VT_M; e += nthreads) {
+            const double2 u = zeta[e];
+            untwist[e >> 6][e & 63] = make_double2(u.x, -u.y);
+        }
+    }
 };
 
 // One exchange of a lane's eight complex values through LDS: written at w + ws s, read at
-// r + rs s.  SEQ: the real parts, then the imaginary parts, through one array (a wave's LDS
+// r + rs s.  SEQ (the wide kernel): the real parts, then the imaginary parts, through one array (a wave's LDS
 // operations complete in order), so the second write overlaps the first read.
 template <bool SEQ>
 __device__ __forceinline__ void vt_exchange(double *re, double *im, double *xr, double *xi, int w, int ws, int r, int rs)
@@ -157,101 +198,87 @@ __device__ __forceinline__ void vt_exchange(double *re, double *im, double *xr, 
     for (int s = 0; s < 8; s++) im[s] = (SEQ ? xr : xi)[r + rs * s];
 }
 
-// Forward transform: layout A in, layout C out.
-// Pass 1's twiddles zeta^r w^(r k) are formed by powers of the lane's w^r from zeta^r
-// (z = {zeta^r, w^r}): seven products instead of eight LDS reads of 16 bytes.
-template <bool SEQ = false, typename T2>
-__device__ __forceinline__ void vt_fwd(double *re, double *im, double *xr, double *xi, const double2 (&z)[2],
-                                       const T2 &t2, int lane)
+// The exchange A<->B in registers: slot bits 2, 1, 0 change places with lane bits 5, 4, 3.
+__device__ __forceinline__ void vt_swap_bit(double &a, double &b, int bit)
 {
-    const int hi = lane >> 3, lo = lane & 7;
-    vt_dft8<-1>(re, im);
-    {
-        double cr = z[0].x, ci = z[0].y;
+    typedef unsigned vt_u2 __attribute__((ext_vector_type(2)));
+    vt_u2 x = __builtin_bit_cast(vt_u2, a), y = __builtin_bit_cast(vt_u2, b);
 #pragma unroll
-        for (int s = 0; s < 8; s++) {
-            vt_cmul(re[s], im[s], cr, ci);
-            if (s < 7) vt_cmul(cr, ci, z[1].x, z[1].y);
+    for (int h = 0; h < 2; h++) {
+        if (bit == 0) {   // lanes 8..15 of a row of 16 take the other's lanes 0..7, and back
+            const unsigned o = x[h];
+            x[h] = __builtin_amdgcn_update_dpp(x[h], y[h], 0x128, 0xf, 0xc, false);
+            y[h] = __builtin_amdgcn_update_dpp(y[h], o, 0x128, 0xf, 0x3, false);
+        } else {
+            const auto r = bit == 2 ? __builtin_amdgcn_permlane32_swap(x[h], y[h], false, false)
+                                    : __builtin_amdgcn_permlane16_swap(x[h], y[h], false, false);
+            x[h] = r[0];
+            y[h] = r[1];
         }
     }
-    vt_exchange<SEQ>(re, im, xr, xi, lane, VT_P1, VT_P1 * hi + lo, 8);
-    vt_dft8<-1>(re, im);
-#pragma unroll
-    for (int s = 1; s < 8; s++) {
-        const double2 t = t2(s, lo);
-        vt_cmul(re[s], im[s], t.x, t.y);
-    }
-    vt_exchange<SEQ>(re, im, xr, xi, VT_P2 * lo + 8 * hi, 1, lane, VT_P2);
-    vt_dft8<-1>(re, im);
+    a = __builtin_bit_cast(double, x);
+    b = __builtin_bit_cast(double, y);
 }
 
-// Inverse transform (unscaled): layout C in, layout A out.
-template <bool SEQ = false, typename T2>
-__device__ __forceinline__ void vt_inv(double *re, double *im, double *xr, double *xi, const double2 (&z)[2],
-                                       const T2 &t2, int lane)
+__device__ __forceinline__ void vt_swap(double *v)
 {
-    const int hi = lane >> 3, lo = lane & 7;
-    vt_dft8<1>(re, im);
 #pragma unroll
-    for (int s = 1; s < 8; s++) {
-        const double2 t = t2(s, lo);
-        vt_cmul(re[s], im[s], t.x, -t.y);
-    }
-    vt_exchange<SEQ>(re, im, xr, xi, lane, VT_P2, VT_P2 * lo + 8 * hi, 1);
-    vt_dft8<1>(re, im);
-    vt_exchange<SEQ>(re, im, xr, xi, VT_P1 * hi + lo, 8, lane, VT_P1);
+    for (int bit = 2; bit >= 0; bit--)
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+            if (!(s & (1 << bit))) vt_swap_bit(v[s], v[s + (1 << bit)], bit);
+}
+
+// The forward twiddles of a lane: passes 2 and 3.
+struct vt_fwd_tw {
+    vt_roots y2, y3;
+    __device__ __forceinline__ vt_fwd_tw(const double2 *zeta, int lane)
+        : y2(vt_roots::at<-1>(zeta, 8 - 32 * (lane >> 3))),
+          y3(vt_roots::at<-1>(zeta, 1 - 4 * ((lane >> 3) + 8 * (lane & 7))))
     {
-        double cr = z[0].x, ci = z[0].y;
-#pragma unroll
-        for (int s = 0; s < 8; s++) {
-            vt_cmul(re[s], im[s], cr, -ci);
-            if (s < 7) vt_cmul(cr, ci, z[1].x, z[1].y);
-        }
     }
-    vt_dft8<1>(re, im);
-}
-
-// {zeta^r, w^r} of lane r from the pass-1 table (w^r = t1[64 + r] conj(t1[r]), |zeta^r| = 1).
-__device__ __forceinline__ void vt_lane_roots(double2 (&z)[2], const double2 *t1, int lane)
-{
-    const double2 a = t1[lane], b = t1[64 + lane];
-    z[0] = a;
-    double r = b.x, i = b.y;
-    vt_cmul(r, i, a.x, -a.y);
-    z[1] = make_double2(r, i);
-}
-
-// The slot factors c_s = zeta^(64 s) = e^(i pi s / 16), correctly rounded (uniform
-// constants, no loads): applied to the forward input, conjugated to the inverse output.
-__device__ constexpr double VT_CS[8][2] = {
-    {1.0, 0.0},
-    {0x1.f6297cff75cb0p-1, 0x1.8f8b83c69a60bp-3},
-    {0x1.d906bcf328d46p-1, 0x1.87de2a6aea963p-2},
-    {0x1.a9b66290ea1a3p-1, 0x1.1c73b39ae68c8p-1},
-    {0x1.6a09e667f3bcdp-1, 0x1.6a09e667f3bcdp-1},
-    {0x1.1c73b39ae68c8p-1, 0x1.a9b66290ea1a3p-1},
-    {0x1.87de2a6aea963p-2, 0x1.d906bcf328d46p-1},
-    {0x1.8f8b83c69a60bp-3, 0x1.f6297cff75cb0p-1},
 };
 
-__device__ __forceinline__ void vt_slot_twist(double *re, double *im, bool conj)
+// Forward transform: layout A in (untwisted), layout C out.
+template <bool SEQ = false>
+__device__ __forceinline__ void vt_fwd(double *re, double *im, double *xr, double *xi, const vt_fwd_tw &t, int lane)
 {
-#pragma unroll
-    for (int s = 1; s < 8; s++) vt_cmul(re[s], im[s], VT_CS[s][0], conj ? -VT_CS[s][1] : VT_CS[s][1]);
+    // y_1 = e^(i pi / 16), correctly rounded (uniform constants, no loads)
+    const vt_roots y1 = {{0x1.6a09e667f3bcdp-1, 0x1.6a09e667f3bcdp-1}, {0x1.d906bcf328d46p-1, 0x1.87de2a6aea963p-2},
+                         {0x1.f6297cff75cb0p-1, 0x1.8f8b83c69a60bp-3}, {0x1.a9b66290ea1a3p-1, -0x1.1c73b39ae68c8p-1}};
+    const int hi = lane >> 3, lo = lane & 7;
+    vt_pass<-1>(re, im, y1);
+    if (SEQ) {
+        vt_exchange<true>(re, im, xr, xi, lane, VT_P1, VT_P1 * hi + lo, 8);
+    } else {
+        vt_swap(re);
+        vt_swap(im);
+    }
+    vt_pass<-1>(re, im, t.y2);
+    vt_exchange<SEQ>(re, im, xr, xi, VT_P2 * lo + 8 * hi, 1, lane, VT_P2);
+    vt_pass<-1>(re, im, t.y3);
 }
 
-// Layout A input of a polynomial given by its coefficients as signed 32-bit values:
-// lane r, slot s holds (p_j + i p_(j+M)) c_s, j = 64 s + r (the lane's twist factor
-// comes with pass 1).
-__device__ __forceinline__ void vt_fold(double *re, double *im, const uint32_t *p, int lane)
+// Inverse transform (unscaled): layout C in, layout A out (untwisted).
+template <bool SEQ = false>
+__device__ __forceinline__ void vt_inv(double *re, double *im, double *xr, double *xi, const vt_inv_tw &t, int lane)
 {
+    const int hi = lane >> 3, lo = lane & 7;
+    vt_dft8<1>(re, im);
+    vt_exchange<SEQ>(re, im, xr, xi, lane, VT_P2, VT_P2 * lo + 8 * hi, 1);
+    vt_pass<1>(re, im, {t.y2[0][lo], t.y2[1][lo], t.y2[2][lo], t.y2[3][lo]});
+    if (SEQ) {
+        vt_exchange<true>(re, im, xr, xi, VT_P1 * hi + lo, 8, lane, VT_P1);
+    } else {
+        vt_swap(re);
+        vt_swap(im);
+    }
+    vt_pass<1>(re, im, {t.y3[0][lane], t.y3[1][lane], t.y3[2][lane], t.y3[3][lane]});
 #pragma unroll
     for (int s = 0; s < 8; s++) {
-        const int j = 64 * s + lane;
-        re[s] = (double)(int32_t)p[j];
-        im[s] = (double)(int32_t)p[j + VT_M];
+        const double2 u = t.untwist[s][lane];
+        vt_cmul(re[s], im[s], u.x, u.y);
     }
-    vt_slot_twist(re, im, false);
 }
 
 // x mod 2^32 of an integer-valued double with |x| < 2^51 (1.5 * 2^52 puts the
@@ -298,17 +325,18 @@ __global__ void __launch_bounds__(256) k_torus_fft(const uint32_t *__restrict__ 
                                                    const double2 *__restrict__ consts, uint64_t count, int natural)
 {
     __shared__ double lds[4][2][VT_XS];
-    __shared__ double2 t1[VT_T1], t2[VT_T2];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    vt_fill_tw(t1, t2, consts, threadIdx.x, 256);
-    __syncthreads();
     const uint64_t poly = (uint64_t)blockIdx.x * 4 + w;
     if (poly >= count) return;   // whole waves leave; the exchanges are wave-private
-    double2 z[2];
-    vt_lane_roots(z, t1, lane);
+    const vt_fwd_tw tw(consts, lane);
+    const uint32_t *p = in + poly * VT_N;
     double re[8], im[8];
-    vt_fold(re, im, in + poly * VT_N, lane);
-    vt_fwd(re, im, lds[w][0], lds[w][1], z, vt_t2_lds{t2}, lane);
+#pragma unroll
+    for (int s = 0; s < 8; s++) {   // p_j + i p_(j+M), j = 64 s + lane
+        re[s] = (double)(int32_t)p[64 * s + lane];
+        im[s] = (double)(int32_t)p[64 * s + lane + VT_M];
+    }
+    vt_fwd(re, im, lds[w][0], lds[w][1], tw, lane);
     double2 *o = out + poly * VT_M;
     const double scale = natural ? 1.0 : 1.0 / VT_M;
 #pragma unroll
@@ -349,6 +377,7 @@ __global__ void __launch_bounds__(128 * ELL, 2) k_torus_blind_rotate_wide(vt_br_
     constexpr int NW = 2 * ELL;
     __shared__ uint32_t acc[2][VT_N];
     __shared__ double2 area[2 * (NW - 1)][VT_M];
+    __shared__ vt_inv_tw itw;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int l = w >> 1, mine = w == 1;   // level (of component w & 1); the component an owner wave keeps
     const uint64_t k = blockIdx.x;
@@ -359,11 +388,8 @@ __global__ void __launch_bounds__(128 * ELL, 2) k_torus_blind_rotate_wide(vt_br_
     auto part = [&](int o, int v) -> double2 * { return area[o * (NW - 1) + (v < o ? v : v - 1)]; };
     double *xs = reinterpret_cast<double *>(part(w == 0 ? 1 : 0, w));
     double *xi = reinterpret_cast<double *>(part(w & 1, NW - 1 - (w & 1) * (NW == 2)));   // read by wave w < 2 only
-    vt_t2_reg t2;
-#pragma unroll
-    for (int s = 0; s < 8; s++) t2.t[s] = A.consts[512 + 8 * s + (lane & 7)];
-    double2 z[2];
-    vt_lane_roots(z, A.consts, lane);
+    const vt_fwd_tw tw(A.consts, lane);
+    itw.fill(A.consts, threadIdx.x, 128 * ELL);   // read by waves 0 and 1 after the first barrier
 
     // acc = (0, X^-rot_b * tv): rot_b from b + floor(2^32 / (4 torus_base)) (cggi16.py:60-71)
     const uint32_t rot_b = vt_mod_switch((uint64_t)in[A.n] + A.offset, shift, two_n);
@@ -421,8 +447,7 @@ __global__ void __launch_bounds__(128 * ELL, 2) k_torus_blind_rotate_wide(vt_br_
             fr[s] = (double)(int)__builtin_amdgcn_sbfe((int)yc[64 * s + lane], sh, B);
             fi[s] = (double)(int)__builtin_amdgcn_sbfe((int)yc[64 * s + lane + VT_M], sh, B);
         }
-        vt_slot_twist(fr, fi, false);
-        vt_fwd<true>(fr, fi, xs, nullptr, z, t2, lane);
+        vt_fwd<true>(fr, fi, xs, nullptr, tw, lane);
         vh_wave_sync();
         double re[8], im[8];
 #pragma unroll
@@ -451,8 +476,7 @@ __global__ void __launch_bounds__(128 * ELL, 2) k_torus_blind_rotate_wide(vt_br_
                     im[s] += p.y;
                 }
             }
-            vt_inv<true>(re, im, xi, nullptr, z, t2, lane);
-            vt_slot_twist(re, im, true);
+            vt_inv<true>(re, im, xi, nullptr, itw, lane);
 #pragma unroll
             for (int s = 0; s < 8; s++) {   // the key carries the 1/M of the inverse
                 own[s] += vt_round_u32(re[s]);
@@ -492,7 +516,7 @@ __global__ void __launch_bounds__(128, 2) k_torus_blind_rotate(vt_br_args A)
 {
     __shared__ uint32_t acc[2][VT_N];
     __shared__ double lds[2][2][VT_XS];
-    __shared__ double2 t1[VT_T1], t2[VT_T2];
+    __shared__ vt_inv_tw itw;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const uint64_t k = blockIdx.x;
     const uint32_t *in = A.lwe + k * (uint64_t)(A.n + 1);
@@ -500,7 +524,8 @@ __global__ void __launch_bounds__(128, 2) k_torus_blind_rotate(vt_br_args A)
     const int shift = 32 - 11;   // log2(2^32 / 2N)
     double *xr = lds[w][0], *xi = lds[w][1];
 
-    vt_fill_tw(t1, t2, A.consts, threadIdx.x, 128);
+    itw.fill(A.consts, threadIdx.x, 128);
+    const vt_fwd_tw tw(A.consts, lane);
 
     // acc = (0, X^-rot_b * tv): rot_b from b + floor(2^32 / (4 torus_base)) (cggi16.py:60-71)
     const uint32_t rot_b = vt_mod_switch((uint64_t)in[A.n] + A.offset, shift, two_n);
@@ -508,8 +533,6 @@ __global__ void __launch_bounds__(128, 2) k_torus_blind_rotate(vt_br_args A)
     uint32_t *mine = acc[w];
     for (int j = lane; j < VT_N; j += 64) mine[j] = w == 0 ? 0u : vt_rot(A.tv, j, rot_tv);
     __syncthreads();
-    double2 z[2];
-    vt_lane_roots(z, t1, lane);
 
     // Digits: with y = x + dec_off, field_l = (y >> sh_l) mod 2^B and d_l = field_l - 2^(B-1),
     // which is the B-bit sign extension of field_l ^ 2^(B-1): one xor per coefficient, then
@@ -552,8 +575,7 @@ __global__ void __launch_bounds__(128, 2) k_torus_blind_rotate(vt_br_args A)
                 re[s] = (double)(int)__builtin_amdgcn_sbfe((int)dlo[s], sh, B);
                 im[s] = (double)(int)__builtin_amdgcn_sbfe((int)dhi[s], sh, B);
             }
-            vt_slot_twist(re, im, false);
-            vt_fwd(re, im, xr, xi, z, vt_t2_lds{t2}, lane);
+            vt_fwd(re, im, xr, xi, tw, lane);
 #pragma unroll
             for (int s = 0; s < 8; s++) {
                 const double2 ko = kor[s], kx = kxr[s];
@@ -582,8 +604,7 @@ __global__ void __launch_bounds__(128, 2) k_torus_blind_rotate(vt_br_args A)
             im[s] = poi[s] + yi[s * 64 + lane];
         }
         __syncthreads();
-        vt_inv(re, im, xr, xi, z, vt_t2_lds{t2}, lane);
-        vt_slot_twist(re, im, true);
+        vt_inv(re, im, xr, xi, itw, lane);
 #pragma unroll
         for (int s = 0; s < 8; s++) {   // the key carries the 1/M of the inverse
             const int j = 64 * s + lane;
@@ -611,9 +632,10 @@ hipError_t vh_launch_torus_blind_rotate(hipStream_t st, const vt_br_args &A, uin
 {
     if (!count) return hipSuccess;
     // Up to one sample per CU the levels of both components run side by side: 3 samples at
-    // n = 630, 3 levels take 2.61 ms against 3.39 ms, 256 take 2.77 against 3.60.  From two samples
-    // per CU on the chip is full of FP64 work either way, and the two-wave form has less LDS
-    // traffic for the partial sums (400 samples: 5.1 ms; 1024: 6.2 ms).
+    // n = 630, 3 levels take 2.50 ms and 256 take 2.62 ms; the two-wave form takes 4.8 ms for 257, as
+    // long as for fewer.  From two samples per CU on the wide form would need two rounds (5.2 ms),
+    // the two-wave form has 512 side by side in 5.0 ms and 1024 in 6.1 ms, where 72% of the
+    // issue slots hold vector instructions.
     const dim3 grid((unsigned)count);
     const bool wide = count <= cus;
 #define VT_BR(EE)                                                                                       \
