@@ -442,6 +442,50 @@ def test_ntt_mul_intt_prime_widths(lib, N, widths, split):
         pool.free(p)
 
 
+@pytest.mark.parametrize("split", [1, 2, 4, 8])
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64, 65])
+def test_work_lists_by_length(lib, rows, split):
+    """Transforms, products and wrap-aware products whose row lists are just within and just past the
+    sizes passed in kernel arguments, limbs of both arithmetics, against the oracle (exact)."""
+    N, L = 512 * split, 2 if rows % 2 == 0 else 1
+    count, primes = rows // L, []
+    for b in (50, 60)[:L]:
+        primes.append(int(O.lib().o_next_special_prime(1 << b, 512, 1)) if b > 50
+                      else O.gen_prime(2 * N // split, b, primes))
+    pool, c, m = rt.Pool(N, primes, split), O.Ctx(N, primes, split), (1 << L) - 1
+    rng = np.random.default_rng(rows * 8 + split)
+    print(f"[lists] rows={rows} split={split}", flush=True)
+    xs = [rt.random_rows(rng, primes, N) for _ in range(count)]
+    ys = [rt.random_rows(rng, primes, N) for _ in range(count)]
+    px, py = [pool.poly(x) for x in xs], [pool.poly(y) for y in ys]
+    pz = [pool.poly() for _ in range(count)]
+    arr = rt._native.voidp_array
+    lib.vfhe_hip_ntt_mul_intt_batch(arr(pz), arr(px), arr(py), count)
+    lib.vfhe_hip_ntt_batch(arr(px), count, 0)
+    lib.vfhe_hip_ntt_batch(arr(py), count, 0)
+    for k in range(count):
+        a, b, z = np.zeros_like(xs[k]), np.zeros_like(xs[k]), np.zeros_like(xs[k])
+        c.to_ntt(a, xs[k], m)
+        c.to_ntt(b, ys[k], m)
+        c.mul(z, a, m, b, m, 0)
+        assert np.array_equal(pool.read(px[k]), a), k
+        for mode, fn in enumerate((lib.polynomial_mul_RNS_polynomial, lib.polynomial_mul_addto_RNS_polynomial,
+                                   lib.polynomial_mul_subto_RNS_polynomial)):
+            if k or split == 1:   # one polynomial is enough for the single products
+                break
+            out, ref = pool.poly(xs[0]), xs[0].copy()
+            fn(out, px[0], py[0])
+            c.mul(ref, a, m, b, m, mode)
+            assert np.array_equal(pool.read(out), ref), mode
+            pool.free(out)
+        c.to_coeff(z, z, m)
+        assert np.array_equal(pool.read(pz[k]), z), k
+    lib.vfhe_hip_ntt_batch(arr(px), count, 1)
+    assert all(np.array_equal(pool.read(p), x) for p, x in zip(px, xs))
+    for p in px + py + pz:
+        pool.free(p)
+
+
 @pytest.mark.slow
 def test_ntt_mul_intt_batch64_config2(lib):
     """The benchmarked fused-product batch: 64 pairs at N = 2^16, L = 24 in one call.  Every product

@@ -61,6 +61,28 @@ struct vh_item {
     uint64_t scalar_sh;   // Shoup companion of `scalar` when used as a multiplier
 };
 
+// A work list: up to CAP items travel in the kernel's arguments, longer ones (and those of graph
+// plans, which are refreshed in place) are read from memory.  A list in host memory costs a
+// kernel 1.5 to 3 us before its first load; CAP items cost the launch CAP * 48 bytes of arguments.
+template <unsigned CAP> struct vh_items_t {
+    const vh_item *p;   // null: the items are in v
+    vh_item v[CAP];
+    __device__ __forceinline__ vh_item operator[](unsigned i) const
+    {
+        if (p) return p[i];
+        return v[i];
+    }
+};
+constexpr unsigned VH_INLINE_ITEMS = 64;
+typedef vh_items_t<VH_INLINE_ITEMS> vh_items;
+template <unsigned CAP> static inline vh_items_t<CAP> vh_items_cut(const vh_items &w, unsigned n)   // p set or n <= CAP
+{
+    vh_items_t<CAP> r;
+    r.p = w.p;
+    if (!w.p) for (unsigned i = 0; i < n; i++) r.v[i] = w.v[i];
+    return r;
+}
+
 // Global address space: pointers read from work lists are otherwise generic
 // (flat) pointers, whose loads wait on both the vector and the LDS counters.
 #define VH_GLOBAL __attribute__((address_space(1)))

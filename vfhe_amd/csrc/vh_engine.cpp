@@ -313,6 +313,17 @@ template <typename T> static T *vh_stage_vec(const std::vector<T> &v)
     return reinterpret_cast<T *>(vh_stage(v.data(), v.size() * sizeof(T)));
 }
 
+// A work list for the kernels that take one by value: short ones travel in the kernel's arguments.
+// A plan refreshes its lists in place and a call without allocations copies its own, so both stay staged.
+static vh_items vh_work(const std::vector<vh_item> &v)
+{
+    vh_items w;
+    w.p = nullptr;
+    if (v.size() <= VH_INLINE_ITEMS && g_cap == VH_CAP_OFF && !g_na_base) memcpy(w.v, v.data(), v.size() * sizeof(vh_item));
+    else w.p = vh_stage_vec(v);
+    return w;
+}
+
 // ---------------------------------------------------------------------------
 // Launch profiler: when on, every kernel launch is bracketed by two HIP events
 // on the engine stream and its duration is summed per kernel family.
@@ -771,6 +782,16 @@ static int col_wide(unsigned items, int logn)
 enum { VH_NTT_WIDE = 0, VH_NTT_FP64 = 1, VH_NTT_INT = 2 };
 static int ntt_kind(const vh_limb &h) { return h.fp64 ? VH_NTT_FP64 : h.q < (1ULL << 62) ? VH_NTT_INT : VH_NTT_WIDE; }
 
+static bool ntt_is_small(int kind, uint64_t n) { return kind != VH_NTT_WIDE && n >= 512 && n <= 4096 && OPT.ntt_small; }
+static void ntt_small_launch(const vh_items &items, unsigned cnt, const vh_limb *d_limbs, int kind, uint64_t n, int dir)
+{
+    // whole transforms in registers, 4096/N of them per workgroup
+    const int fp = kind == VH_NTT_FP64;
+    vh_prof_scope ps_(fp ? VH_PROF_NTT_FP64 : VH_PROF_NTT_INT);
+    VH_LAUNCH(vh_launch_ntt_small(S(), items, cnt, d_limbs, dir, ilog2(n), fp));
+    g_ntt_small_launches++;
+}
+
 // Launches the transforms of `cnt` staged work items (device list d_items, all of one
 // arithmetic, ntt_kind) of n-point rows, direction dir.
 static void ntt_dispatch(const vh_item *d_items, unsigned cnt, const vh_limb *d_limbs, int kind, uint64_t n, int dir)
@@ -817,11 +838,10 @@ static void ntt_dispatch(const vh_item *d_items, unsigned cnt, const vh_limb *d_
                 { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16(S(), ci, cc, d_limbs, 1, logn, 0, R1, 1, 0, 1)); }
             }
         }
-    } else if (kind != VH_NTT_WIDE && logn >= 9 && logn <= 12 && OPT.ntt_small) {
-        // whole transforms in registers, 4096/N of them per workgroup
-        vh_prof_scope ps_(fp ? VH_PROF_NTT_FP64 : VH_PROF_NTT_INT);
-        VH_LAUNCH(vh_launch_ntt_small(S(), d_items, cnt, d_limbs, dir, logn, fp));
-        g_ntt_small_launches++;
+    } else if (ntt_is_small(kind, n)) {
+        vh_items w;
+        w.p = d_items;
+        ntt_small_launch(w, cnt, d_limbs, kind, n, dir);
     } else if (kind == VH_NTT_INT && logn >= 13 && logn <= 16) {
         // two register passes, column then row (inverse: row then column)
         for (int pass = 0; pass < 2; pass++) {
@@ -858,7 +878,8 @@ static void run_ntt(std::vector<vh_item> &items, const vh_limb *d_limbs, const v
         for (size_t off = 0; off < v.size(); off += VH_MAX_GRID_Y) {
             const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, v.size() - off);
             std::vector<vh_item> chunk(v.begin() + off, v.begin() + off + cnt);
-            ntt_dispatch(vh_stage_vec(chunk), cnt, d_limbs, kind, n, dir);
+            if (ntt_is_small(kind, n)) ntt_small_launch(vh_work(chunk), cnt, d_limbs, kind, n, dir);
+            else ntt_dispatch(vh_stage_vec(chunk), cnt, d_limbs, kind, n, dir);
         }
     }
 }
@@ -1523,7 +1544,7 @@ static void run_muls(const std::vector<vh_mulreq> &reqs, int mode)
             std::vector<vh_item> chunk(items.begin() + off, items.begin() + off + cnt);
             {
                 vh_prof_scope ps_(VH_PROF_ELTWISE);
-                VH_LAUNCH(vh_launch_split_mul(S(), vh_stage_vec(chunk), cnt, P->d_limbs, mode, P->n, t->split_degree));
+                VH_LAUNCH(vh_launch_split_mul(S(), vh_work(chunk), cnt, P->d_limbs, mode, P->n, t->split_degree));
             }
         }
     }
@@ -2546,7 +2567,7 @@ static void gadget_batch(const std::vector<RNS_MLWE> &outs, const std::vector<st
                             chunk.push_back(it);
                         }
                     vh_prof_scope ps_(VH_PROF_ELTWISE);
-                    VH_LAUNCH(vh_launch_split_mul(S(), vh_stage_vec(chunk), (unsigned)chunk.size(), P->d_limbs,
+                    VH_LAUNCH(vh_launch_split_mul(S(), vh_work(chunk), (unsigned)chunk.size(), P->d_limbs,
                                                  add ? 1 : 2, P->n, t->split_degree));
                 }
             }
@@ -3940,7 +3961,7 @@ static void ntt_mul_intt(RNS_Polynomial *z, RNS_Polynomial *x, RNS_Polynomial *y
                 const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, items.size() - off);
                 std::vector<vh_item> chunk(items.begin() + off, items.begin() + off + cnt);
                 vh_prof_scope ps_(kind == VH_NTT_FP64 ? VH_PROF_NTT_FP64 : VH_PROF_NTT_INT);
-                VH_LAUNCH(vh_launch_product_small(S(), vh_stage_vec(chunk), cnt, P->d_limbs, logn, kind == VH_NTT_FP64));
+                VH_LAUNCH(vh_launch_product_small(S(), vh_work(chunk), cnt, P->d_limbs, logn, kind == VH_NTT_FP64));
             }
         }
         return;
@@ -3981,7 +4002,7 @@ static void ntt_mul_intt(RNS_Polynomial *z, RNS_Polynomial *x, RNS_Polynomial *y
             const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, mul.size() - off);
             std::vector<vh_item> chunk(mul.begin() + off, mul.begin() + off + cnt);
             vh_prof_scope ps_(VH_PROF_ELTWISE);
-            VH_LAUNCH(vh_launch_split_mul(S(), vh_stage_vec(chunk), cnt, P->d_limbs, 0, P->n, split));
+            VH_LAUNCH(vh_launch_split_mul(S(), vh_work(chunk), cnt, P->d_limbs, 0, P->n, split));
         }
     }
     run_ntt(inv, P->d_limbs, P->h_limbs.data(), P->n, 1);

@@ -92,9 +92,9 @@ struct vh_mac_job {
 // Whole transforms of N = 2^9 .. 2^12 (reads it.src, writes it.dst), and whole negacyclic products
 // z = INTT(NTT(x) NTT(y)) (x it.src, y it.src2, z it.dst), in registers.  fp: every limb FP64,
 // else every limb integer with q < 2^62.
-hipError_t vh_launch_ntt_small(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, int dir,
+hipError_t vh_launch_ntt_small(hipStream_t st, const vh_items &items, unsigned nitems, const vh_limb *limbs, int dir,
                                int logn, int fp);
-hipError_t vh_launch_product_small(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs,
+hipError_t vh_launch_product_small(hipStream_t st, const vh_items &items, unsigned nitems, const vh_limb *limbs,
                                    int logn, int fp);
 // Integer path (q < 2^62), N = 2^13 .. 2^16: one pass of a transform (dir 0: col then row, dir 1: row
 // then col; the first pass reads it.src, the second works in it.dst), and the product's middle step.
@@ -179,7 +179,7 @@ hipError_t vh_launch_tensor1(hipStream_t st, const vh_tensor_job *jobs, unsigned
                              uint64_t n);
 hipError_t vh_launch_eltwise(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs,
                              int op, uint64_t n);
-hipError_t vh_launch_split_mul(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs,
+hipError_t vh_launch_split_mul(hipStream_t st, const vh_items &items, unsigned nitems, const vh_limb *limbs,
                                int mode, uint64_t n, uint64_t S);
 // cdown: K x nl division constants of the special primes; cresc: 1 x nl of the rescale prime.
 hipError_t vh_launch_moddown_rescale(hipStream_t st, const vh_mdr_job *jobs, unsigned njobs, const vh_limb *limbs,

@@ -709,29 +709,52 @@ k_eltwise(const vh_item *__restrict__ items, const vh_limb *__restrict__ limbs, 
 // split_degree > 1): out block d = sum_{j+k = d (mod S)} in1_j * in2_k * (w if
 // j + k >= S).  mode 0: =, 1: +=, 2: -=.  One thread per (block position x,
 // output block d); items: src = in1 row, src2 = in2 row, dst = out row, aux = S,
-// scalar = device address of the w row.
+// scalar = device address of the w row.  The wrapped products are summed before their one
+// product with w; S = 2 and 4 (compile time) have every operand loaded before the first product.
+// Latency is what a single ring product waits for: 7 limbs of N = 4096 at S = 4 took 7.0 us with
+// runtime indices, a product with w per term and the list read from host memory; 3.8 us now.
 // ---------------------------------------------------------------------------
+template <int SP, unsigned CAP>   // SP: split degree, 0: it.aux
 __global__ void __launch_bounds__(256)
-k_split_mul(const vh_item *__restrict__ items, const vh_limb *__restrict__ limbs, int mode, uint64_t n)
+k_split_mul(const vh_items_t<CAP> items, const vh_limb *__restrict__ limbs, int mode, int logn)
 {
     const vh_item it = items[blockIdx.y];
     const vh_limb L = limbs[it.limb];
     const uint64_t q = L.q, mu = L.mu64;
-    const int S = it.aux;
-    const uint64_t *w = reinterpret_cast<const uint64_t *>(it.scalar);
-    const uint64_t total = n * S;
+    const int S = SP ? SP : (int)it.aux;
+    const VH_GLOBAL uint64_t *w = vh_global(reinterpret_cast<const uint64_t *>(it.scalar));
+    const VH_GLOBAL uint64_t *in1 = vh_global(it.src), *in2 = vh_global(it.src2);
+    VH_GLOBAL uint64_t *out = vh_global(it.dst);
+    const uint64_t total = (uint64_t)S << logn;
     for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t d = e / n, x = e % n;
-        uint64_t acc = 0;
-        for (int j = 0; j < S; j++) {
-            const int k = (int)((d + S - j) % S);
-            uint64_t p = vh_mulmod(vh_reduce64(it.src[j * n + x], q, mu), vh_reduce64(it.src2[k * n + x], q, mu), L);
-            if (j + k >= S) p = vh_mulmod(p, w[x], L);
-            acc = vh_addmod(acc, p, q);
+        const int d = (int)(e >> logn);
+        const uint64_t x = e & (((uint64_t)1 << logn) - 1);
+        uint64_t lo = 0, hi = 0;
+        auto term = [&](uint64_t a, uint64_t b, bool wrap) {
+            const uint64_t p = vh_mulmod(vh_reduce64(a, q, mu), vh_reduce64(b, q, mu), L);
+            lo = vh_addmod(lo, wrap ? 0 : p, q);
+            hi = vh_addmod(hi, wrap ? p : 0, q);
+        };
+        if (SP) {
+            uint64_t a[SP ? SP : 1], b[SP ? SP : 1];
+            const uint64_t wx = w[x];
+#pragma unroll
+            for (int j = 0; j < SP; j++) {
+                a[j] = in1[((uint64_t)j << logn) + x];
+                b[j] = in2[((uint64_t)((d - j) & (SP - 1)) << logn) + x];
+            }
+#pragma unroll
+            for (int j = 0; j < SP; j++) term(a[j], b[j], j > d);
+            if (d + 1 < SP) lo = vh_addmod(lo, vh_mulmod(hi, wx, L), q);
+        } else {
+            for (int j = 0; j < S; j++) term(in1[((uint64_t)j << logn) + x], in2[((uint64_t)((d - j) & (S - 1)) << logn) + x], j > d);
+            if (d + 1 < S) lo = vh_addmod(lo, vh_mulmod(hi, w[x], L), q);
         }
-        uint64_t o = it.dst[d * n + x];
-        it.dst[d * n + x] = mode == 0 ? acc : (mode == 1 ? vh_addmod(vh_reduce64(o, q, mu), acc, q)
-                                                         : vh_submod(vh_reduce64(o, q, mu), acc, q));
+        if (mode) {
+            const uint64_t o = vh_reduce64(out[e], q, mu);
+            lo = mode == 1 ? vh_addmod(o, lo, q) : vh_submod(o, lo, q);
+        }
+        out[e] = lo;
     }
 }
 
@@ -1219,10 +1242,19 @@ hipError_t vh_launch_eltwise(hipStream_t st, const vh_item *items, unsigned nite
     return hipGetLastError();
 }
 
-hipError_t vh_launch_split_mul(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs,
+hipError_t vh_launch_split_mul(hipStream_t st, const vh_items &items, unsigned nitems, const vh_limb *limbs,
                                int mode, uint64_t n, uint64_t S)
 {
-    VH_KL(k_split_mul, dim3(vh_blocks(n * S, 256, 64), nitems), dim3(256), 0, st, items, limbs, mode, n);
+    const int logn = 63 - __builtin_clzll(n);   // n and S are powers of two (new_incomplete_ntt_list)
+    const dim3 grid(vh_blocks(n * S, 256, 64), nitems);
+    auto go = [&](const auto &list) {
+        constexpr unsigned CAP = sizeof(list.v) / sizeof(vh_item);
+        if (S == 2) VH_KL((k_split_mul<2, CAP>), grid, dim3(256), 0, st, list, limbs, mode, logn);
+        else if (S == 4) VH_KL((k_split_mul<4, CAP>), grid, dim3(256), 0, st, list, limbs, mode, logn);
+        else VH_KL((k_split_mul<0, CAP>), grid, dim3(256), 0, st, list, limbs, mode, logn);
+    };
+    if (items.p || nitems <= 16) go(vh_items_cut<16>(items, nitems));
+    else go(items);
     return hipGetLastError();
 }
 

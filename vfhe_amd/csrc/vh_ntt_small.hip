@@ -9,9 +9,9 @@
 // the stride ownership (whole 128-byte runs per instruction); the forward pass regroups its
 // output through LDS for that.
 // ---------------------------------------------------------------------------
-template <int DIR, int LOGN, typename AR>
+template <int DIR, int LOGN, typename AR, unsigned CAP>
 __global__ void __launch_bounds__(256)
-k_ntt_small(const vh_item *__restrict__ items, unsigned nitems, const vh_limb *__restrict__ limbs)
+k_ntt_small(const vh_items_t<CAP> items, unsigned nitems, const vh_limb *__restrict__ limbs)
 {
     using R = vh_reg_ntt<LOGN>;
     using V = typename AR::V;
@@ -24,7 +24,7 @@ k_ntt_small(const vh_item *__restrict__ items, unsigned nitems, const vh_limb *_
     const bool live = idx < nitems;
     // a slot past the end transforms the last item again (every thread reaches the
     // barriers) and stores nothing
-    const vh_item &it = items[live ? idx : nitems - 1];
+    const vh_item it = items[live ? idx : nitems - 1];
     const vh_limb &L = limbs[it.limb];
     const AR ar(L, DIR);
     V *lds = lds_all + slot * PAD;
@@ -58,10 +58,10 @@ k_ntt_small(const vh_item *__restrict__ items, unsigned nitems, const vh_limb *_
 // transforms, the product and the inverse stay in registers.  One launch and 24 N bytes per row
 // where separate transforms and a product take 88 N bytes, three launches and temporaries.
 // 37 pairs x 3 limbs of N = 2048: 189 us a call (24 us of it kernels, the rest a temporary
-// polynomial per pair) -> 24 us.  Bound there by latency, at large batches by HBM.
+// polynomial per pair) -> 21 us.  Bound there by latency, at large batches by HBM.
 template <int LOGN, typename AR>
 __global__ void __launch_bounds__(256, 2)
-k_product_small(const vh_item *__restrict__ items, unsigned nitems, const vh_limb *__restrict__ limbs)
+k_product_small(const vh_items items, unsigned nitems, const vh_limb *__restrict__ limbs)
 {
     using R = vh_reg_ntt<LOGN>;
     using V = typename AR::V;
@@ -71,7 +71,7 @@ k_product_small(const vh_item *__restrict__ items, unsigned nitems, const vh_lim
     const int tid = threadIdx.x, slot = tid / T, t = tid % T;
     const unsigned idx = blockIdx.x * PER + slot;
     const bool live = idx < nitems;
-    const vh_item &it = items[live ? idx : nitems - 1];
+    const vh_item it = items[live ? idx : nitems - 1];
     const vh_limb &L = limbs[it.limb];
     const AR fw(L, 0), iv(L, 1);
     V *lds = lds_all + slot * PAD;
@@ -259,24 +259,34 @@ k_ntt16i_row_mul(const vh_item *__restrict__ items, const vh_limb *__restrict__ 
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-hipError_t vh_launch_ntt_small(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, int dir,
+// Lists in the arguments (vh_items_t) by length: 16 polynomials x 4 limbs of N = 4096 took 11.1 us with the
+// list in host memory, 7.6 us so.  The argument block grows with the list it can hold because
+// the launch pays for it: a single ring product, two launches of 7 and 28 rows, takes 22.5 us with
+// 3 KiB of arguments for each and 19.5 us with these sizes (21.8 us with lists in host memory).
+template <int LOGN, typename AR, unsigned CAP>
+static void vh_ntt_small_go(hipStream_t st, const vh_items_t<CAP> &items, unsigned nitems, const vh_limb *limbs, int dir)
+{
+    const unsigned per = 4096u >> LOGN, nb = (nitems + per - 1) / per;
+    if (dir == 0) VH_KL((k_ntt_small<0, LOGN, AR, CAP>), dim3(nb), dim3(256), 0, st, items, nitems, limbs);
+    else VH_KL((k_ntt_small<1, LOGN, AR, CAP>), dim3(nb), dim3(256), 0, st, items, nitems, limbs);
+}
+
+hipError_t vh_launch_ntt_small(hipStream_t st, const vh_items &items, unsigned nitems, const vh_limb *limbs, int dir,
                                int logn, int fp)
 {
     if (logn < 9 || logn > 12 || nitems == 0) return hipErrorInvalidValue;
-    const unsigned per = 4096u >> logn, nb = (nitems + per - 1) / per;
-#define VH_SMALL(LG)                                                                                                \
-    case LG:                                                                                                        \
-        if (fp && dir == 0) VH_KL((k_ntt_small<0, LG, vh_ar_fp>), dim3(nb), dim3(256), 0, st, items, nitems, limbs); \
-        else if (fp) VH_KL((k_ntt_small<1, LG, vh_ar_fp>), dim3(nb), dim3(256), 0, st, items, nitems, limbs);        \
-        else if (dir == 0) VH_KL((k_ntt_small<0, LG, vh_ar_int>), dim3(nb), dim3(256), 0, st, items, nitems, limbs); \
-        else VH_KL((k_ntt_small<1, LG, vh_ar_int>), dim3(nb), dim3(256), 0, st, items, nitems, limbs);               \
-        break;
-    switch (logn) { VH_SMALL(9) VH_SMALL(10) VH_SMALL(11) VH_SMALL(12) }
+#define VH_SMALL(LG, AR)                                                                                    \
+        if (items.p || nitems <= 16) vh_ntt_small_go<LG, AR>(st, vh_items_cut<16>(items, nitems), nitems, limbs, dir); \
+        else if (nitems <= 32) vh_ntt_small_go<LG, AR>(st, vh_items_cut<32>(items, nitems), nitems, limbs, dir);       \
+        else vh_ntt_small_go<LG, AR>(st, items, nitems, limbs, dir);
+#define VH_SIZE(LG) case LG: if (fp) { VH_SMALL(LG, vh_ar_fp) } else { VH_SMALL(LG, vh_ar_int) } break;
+    switch (logn) { VH_SIZE(9) VH_SIZE(10) VH_SIZE(11) VH_SIZE(12) }
+#undef VH_SIZE
 #undef VH_SMALL
     return hipGetLastError();
 }
 
-hipError_t vh_launch_product_small(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs,
+hipError_t vh_launch_product_small(hipStream_t st, const vh_items &items, unsigned nitems, const vh_limb *limbs,
                                    int logn, int fp)
 {
     if (logn < 9 || logn > 12 || nitems == 0) return hipErrorInvalidValue;
