@@ -486,6 +486,27 @@ def test_work_lists_by_length(lib, rows, split):
         pool.free(p)
 
 
+@pytest.mark.parametrize("rows", [1, 31, 32, 33])
+def test_two_pass_lists_by_length(lib, rows):
+    """Two-pass transforms (N = 8192) of row lists just within and past the 32 rows passed in kernel
+    arguments, both directions, against the oracle (exact)."""
+    N = 8192
+    primes = O.gen_primes(N, [50])
+    pool, c, rng = rt.Pool(N, primes), O.Ctx(N, primes), np.random.default_rng(rows)
+    print(f"[lists] two passes, rows={rows}", flush=True)
+    xs = [rt.random_rows(rng, primes, N) for _ in range(rows)]
+    ps = [pool.poly(x) for x in xs]
+    lib.vfhe_hip_ntt_batch(rt._native.voidp_array(ps), rows, 0)
+    for p, x in zip(ps, xs):
+        ref = np.zeros_like(x)
+        c.to_ntt(ref, x, 1)
+        assert np.array_equal(pool.read(p), ref)
+    lib.vfhe_hip_ntt_batch(rt._native.voidp_array(ps), rows, 1)
+    for p, x in zip(ps, xs):
+        assert np.array_equal(pool.read(p), x)
+        pool.free(p)
+
+
 @pytest.mark.slow
 def test_ntt_mul_intt_batch64_config2(lib):
     """The benchmarked fused-product batch: 64 pairs at N = 2^16, L = 24 in one call.  Every product

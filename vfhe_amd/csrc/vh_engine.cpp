@@ -315,11 +315,11 @@ template <typename T> static T *vh_stage_vec(const std::vector<T> &v)
 
 // A work list for the kernels that take one by value: short ones travel in the kernel's arguments.
 // A plan refreshes its lists in place and a call without allocations copies its own, so both stay staged.
-static vh_items vh_work(const std::vector<vh_item> &v)
+static vh_items vh_work(const std::vector<vh_item> &v, unsigned cap = VH_INLINE_ITEMS)
 {
     vh_items w;
     w.p = nullptr;
-    if (v.size() <= VH_INLINE_ITEMS && g_cap == VH_CAP_OFF && !g_na_base) memcpy(w.v, v.data(), v.size() * sizeof(vh_item));
+    if (v.size() <= cap && g_cap == VH_CAP_OFF && !g_na_base) memcpy(w.v, v.data(), v.size() * sizeof(vh_item));
     else w.p = vh_stage_vec(v);
     return w;
 }
@@ -792,11 +792,22 @@ static void ntt_small_launch(const vh_items &items, unsigned cnt, const vh_limb 
     g_ntt_small_launches++;
 }
 
-// Launches the transforms of `cnt` staged work items (device list d_items, all of one
+static vh_items vh_staged(const vh_item *d) { vh_items w; w.p = d; return w; }
+
+// The longest list ntt_dispatch takes in kernel arguments (0: every list must be staged).
+static unsigned ntt_inline_cap(int kind, uint64_t n)
+{
+    return n >= 8192 && n <= 65536 && kind == VH_NTT_FP64 && OPT.ntt_mode == 2 && C.pipe_blocks > 0 &&
+           OPT.ntt_chunk_mb <= 0 ? VH_PASS_ITEMS : ntt_is_small(kind, n) ? VH_INLINE_ITEMS : 0;
+}
+
+// Launches the transforms of `cnt` work items (device list d_items, all of one
 // arithmetic, ntt_kind) of n-point rows, direction dir.
-static void ntt_dispatch(const vh_item *d_items, unsigned cnt, const vh_limb *d_limbs, int kind, uint64_t n, int dir)
+static void ntt_dispatch(const vh_items &list, unsigned cnt, const vh_limb *d_limbs, int kind, uint64_t n, int dir)
 {
     const int logn = ilog2(n), fp = kind == VH_NTT_FP64;
+    const vh_item *d_items = list.p;   // null: the list is in `list`, at most ntt_inline_cap items
+    VH_REQUIRE(d_items || cnt <= ntt_inline_cap(kind, n));
     if (fp && logn >= 13 && logn <= 16 && OPT.ntt_mode == 1 && C.xcd_ok) {
         // Persistent kernel: both passes of every transform on one XCD, the
         // intermediate exchanged through that XCD's L2.
@@ -822,13 +833,14 @@ static void ntt_dispatch(const vh_item *d_items, unsigned cnt, const vh_limb *d_
             const unsigned cc = std::min(per, cnt - c0);
             const vh_item *ci = d_items + c0;
             if (pipe) {
+                const vh_items w = d_items ? vh_staged(ci) : list;   // no sub-batches without staging
                 auto nb = [&](int bit) -> unsigned { return (OPT.ntt_tile_grid >> bit) & 1 ? UINT_MAX : C.pipe_blocks; };
                 if (dir == 0) {
-                    { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16p(S(), ci, cc, d_limbs, 0, logn, 0, R1, 1, 1, 0, nb(0), col_wide(cc, logn))); }
-                    { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16p(S(), ci, cc, d_limbs, 0, logn, R1, 8, 0, 0, 1, nb(1))); }
+                    { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16p(S(), w, cc, d_limbs, 0, logn, 0, R1, 1, 1, 0, nb(0), col_wide(cc, logn))); }
+                    { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16p(S(), w, cc, d_limbs, 0, logn, R1, 8, 0, 0, 1, nb(1))); }
                 } else {
-                    { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16p(S(), ci, cc, d_limbs, 1, logn, R1, 8, 0, 1, 0, nb(2))); }
-                    { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16p(S(), ci, cc, d_limbs, 1, logn, 0, R1, 1, 0, 1, nb(3), col_wide(cc, logn))); }
+                    { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16p(S(), w, cc, d_limbs, 1, logn, R1, 8, 0, 1, 0, nb(2))); }
+                    { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16p(S(), w, cc, d_limbs, 1, logn, 0, R1, 1, 0, 1, nb(3), col_wide(cc, logn))); }
                 }
             } else if (dir == 0) {
                 { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16(S(), ci, cc, d_limbs, 0, logn, 0, R1, 1, 1, 0)); }
@@ -839,9 +851,7 @@ static void ntt_dispatch(const vh_item *d_items, unsigned cnt, const vh_limb *d_
             }
         }
     } else if (ntt_is_small(kind, n)) {
-        vh_items w;
-        w.p = d_items;
-        ntt_small_launch(w, cnt, d_limbs, kind, n, dir);
+        ntt_small_launch(list, cnt, d_limbs, kind, n, dir);
     } else if (kind == VH_NTT_INT && logn >= 13 && logn <= 16) {
         // two register passes, column then row (inverse: row then column)
         for (int pass = 0; pass < 2; pass++) {
@@ -878,8 +888,7 @@ static void run_ntt(std::vector<vh_item> &items, const vh_limb *d_limbs, const v
         for (size_t off = 0; off < v.size(); off += VH_MAX_GRID_Y) {
             const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, v.size() - off);
             std::vector<vh_item> chunk(v.begin() + off, v.begin() + off + cnt);
-            if (ntt_is_small(kind, n)) ntt_small_launch(vh_work(chunk), cnt, d_limbs, kind, n, dir);
-            else ntt_dispatch(vh_stage_vec(chunk), cnt, d_limbs, kind, n, dir);
+            ntt_dispatch(vh_work(chunk, ntt_inline_cap(kind, n)), cnt, d_limbs, kind, n, dir);
         }
     }
 }
@@ -2488,7 +2497,7 @@ static void gadget_batch(const std::vector<RNS_MLWE> &outs, const std::vector<st
                 // One tile per workgroup (the grid runs tile-major, so the workgroups in
                 // flight share two or three digit rows, which stay in the L2).
                 if (OPT.ntt_mode == 2 && C.pipe_blocks > 0)
-                    VH_LAUNCH(vh_launch_ntt16p(S(), vh_stage_vec(chunk), cnt, P->d_limbs, 0, logn, 0, logn - 8, 1, 2, 0,
+                    VH_LAUNCH(vh_launch_ntt16p(S(), vh_work(chunk, VH_PASS_ITEMS), cnt, P->d_limbs, 0, logn, 0, logn - 8, 1, 2, 0,
                                               UINT_MAX, col_wide(cnt, logn)));
                 else
                     VH_LAUNCH(vh_launch_ntt16(S(), vh_stage_vec(chunk), cnt, P->d_limbs, 0, logn, 0, logn - 8, 1, 2, 0));
@@ -3543,7 +3552,7 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
             vh_prof_scope ps_(VH_PROF_ELTWISE);
             VH_LAUNCH(vh_launch_eltwise(S(), d_lift + off, cn, P->d_limbs, VH_OP_REDUCE, N));
         });
-        chunks(nt.size(), [&](size_t off, unsigned cn) { ntt_dispatch(d_nt + off, cn, P->d_limbs, kind, N, 0); });
+        chunks(nt.size(), [&](size_t off, unsigned cn) { ntt_dispatch(vh_staged(d_nt + off), cn, P->d_limbs, kind, N, 0); });
         // 3. external product with bk[i]: row (ti, d, c) of the key table
         for (uint64_t d = 0; d < nd; d++) {
             const uint64_t src = d / J.size(), jj = d % J.size();
@@ -3561,7 +3570,7 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
             VH_LAUNCH(vh_launch_keyswitch_mac(S(), d_jobs + off, cn, (unsigned)next, P->d_limbs, d_kptr, N, fp ? 1 : 0));
         });
         // 4. back to coefficient form, round-divided by the special limbs (their rows cleared)
-        chunks(inv.size(), [&](size_t off, unsigned cn) { ntt_dispatch(d_inv + off, cn, P->d_limbs, kind, N, 1); });
+        chunks(inv.size(), [&](size_t off, unsigned cn) { ntt_dispatch(vh_staged(d_inv + off), cn, P->d_limbs, kind, N, 1); });
         if (!divs.empty()) {
             chunks(dj.size(), [&](size_t off, unsigned cn) {
                 vh_prof_scope ps_(VH_PROF_DIVISION);
@@ -3902,22 +3911,22 @@ static void fused_product_launches(std::vector<vh_item> &col, std::vector<vh_ite
         for (size_t off = 0; off < v.size(); off += VH_MAX_GRID_Y) {
             const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, v.size() - off);
             std::vector<vh_item> chunk(v.begin() + off, v.begin() + off + cnt);
-            const vh_item *d = vh_stage_vec(chunk);
+            const bool pipe = OPT.ntt_mode == 2 && C.pipe_blocks > 0;
+            const vh_items d = vh_work(chunk, kind == VH_NTT_FP64 && pipe && which != 1 ? VH_PASS_ITEMS : 0);
             if (kind == VH_NTT_INT) {
                 vh_prof_scope ps_(VH_PROF_NTT_INT);
-                if (which == 1) VH_LAUNCH(vh_launch_ntt16i_row_mul(S(), d, cnt, P->d_limbs, logn));
-                else VH_LAUNCH(vh_launch_ntt16i(S(), d, cnt, P->d_limbs, which == 0 ? 0 : 1, logn, 1));
+                if (which == 1) VH_LAUNCH(vh_launch_ntt16i_row_mul(S(), d.p, cnt, P->d_limbs, logn));
+                else VH_LAUNCH(vh_launch_ntt16i(S(), d.p, cnt, P->d_limbs, which == 0 ? 0 : 1, logn, 1));
                 continue;
             }
             vh_prof_scope ps_(VH_PROF_NTT_FP64);
-            const bool pipe = OPT.ntt_mode == 2 && C.pipe_blocks > 0;
             const unsigned nb0 = (OPT.ntt_tile_grid & 1) ? UINT_MAX : C.pipe_blocks;
             const unsigned nb3 = ((OPT.ntt_tile_grid >> 3) & 1) ? UINT_MAX : C.pipe_blocks;
             if (which == 0 && pipe) VH_LAUNCH(vh_launch_ntt16p(S(), d, cnt, P->d_limbs, 0, logn, 0, R1, 1, 1, 0, nb0, col_wide(cnt, logn)));
-            else if (which == 0) VH_LAUNCH(vh_launch_ntt16(S(), d, cnt, P->d_limbs, 0, logn, 0, R1, 1, 1, 0));
-            else if (which == 1) VH_LAUNCH(vh_launch_row_mul(S(), d, cnt, P->d_limbs, logn));
+            else if (which == 0) VH_LAUNCH(vh_launch_ntt16(S(), d.p, cnt, P->d_limbs, 0, logn, 0, R1, 1, 1, 0));
+            else if (which == 1) VH_LAUNCH(vh_launch_row_mul(S(), d.p, cnt, P->d_limbs, logn));
             else if (pipe) VH_LAUNCH(vh_launch_ntt16p(S(), d, cnt, P->d_limbs, 1, logn, 0, R1, 1, 0, 1, nb3, col_wide(cnt, logn)));
-            else VH_LAUNCH(vh_launch_ntt16(S(), d, cnt, P->d_limbs, 1, logn, 0, R1, 1, 0, 1));
+            else VH_LAUNCH(vh_launch_ntt16(S(), d.p, cnt, P->d_limbs, 1, logn, 0, R1, 1, 0, 1));
         }
     };
     launch(col, 0);

@@ -165,7 +165,7 @@ hipError_t vh_launch_ntt16(hipStream_t st, const vh_item *items, unsigned nitems
 // forward column pass only), nblocks persistent workgroups of 256 threads (at most one per tile);
 // needs vh_limb::rowf_* for row passes.  wide: a column pass runs 512-thread workgroups over
 // twice the columns per tile (nblocks is halved).
-hipError_t vh_launch_ntt16p(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, int dir,
+hipError_t vh_launch_ntt16p(hipStream_t st, const vh_items &items, unsigned nitems, const vh_limb *limbs, int dir,
                             int logn, int s0, int R, int col, int first, int last, unsigned nblocks, int wide = 0);
 int vh_ntt16p_occupancy();
 // Persistent two-pass NTT with per-XCD queues; ctl holds 16 + nitems zeroed uint32 counters.

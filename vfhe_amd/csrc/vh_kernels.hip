@@ -349,9 +349,10 @@ k_ntt16(const vh_item *__restrict__ items, const vh_limb *__restrict__ limbs, in
 // are the same for its 16 threads: thread e < 15 forms twiddle e once per tile
 // into the row's padding slots of the exchange buffer, which no exchange writes.
 // ---------------------------------------------------------------------------
-template <int DIR, int R, bool COL, bool FIRST, bool LAST, bool SHARED = false, int NT = 256>
+// ARGS: vh_items_args has the items, or vh_items_mem and they are in `list`.
+template <int DIR, int R, bool COL, bool FIRST, bool LAST, bool SHARED = false, int NT = 256, typename ARGS = vh_items_mem>
 __global__ void __launch_bounds__(NT, 1024 / NT)
-k_ntt16p(const vh_item *__restrict__ items, const vh_limb *__restrict__ limbs, int logn, int s0,
+k_ntt16p(const vh_item *__restrict__ list, const ARGS args, const vh_limb *__restrict__ limbs, int logn, int s0,
          unsigned tiles_per_item, unsigned ntiles)
 {
     // NT threads: 256, or 512 for a column pass over twice as many columns per tile
@@ -387,7 +388,7 @@ k_ntt16p(const vh_item *__restrict__ items, const vh_limb *__restrict__ limbs, i
     __shared__ double2 rowb[2][G][8];
     double2 fnext = make_double2(0.0, 0.0);
     auto fetch = [&](unsigned uu) {
-        const vh_item &iu = items[uu / tiles_per_item];
+        const vh_item &iu = args.at(list, uu / tiles_per_item);
         const size_t su = (size_t)(uu % tiles_per_item) * G + g;
         if (!COL && t < 8) {   // issued first: landed whenever the data has
             const vh_limb &Lu = limbs[iu.limb];
@@ -409,7 +410,7 @@ k_ntt16p(const vh_item *__restrict__ items, const vh_limb *__restrict__ limbs, i
     unsigned cur_limb = ~0u;
     if (u0 < u1) fetch(u0);
     for (unsigned u = u0; u < u1; u++) {
-        const vh_item &it = items[u / tiles_per_item];
+        const vh_item &it = args.at(list, u / tiles_per_item);
         const vh_limb &L = limbs[it.limb];
         const double q = L.qd, qinv = L.qinv;
         const size_t sub = (size_t)(u % tiles_per_item) * G + g;
@@ -1336,10 +1337,11 @@ hipError_t vh_launch_ntt16(hipStream_t st, const vh_item *items, unsigned nitems
     return hipGetLastError();
 }
 
-hipError_t vh_launch_ntt16p(hipStream_t st, const vh_item *items, unsigned nitems, const vh_limb *limbs, int dir,
+hipError_t vh_launch_ntt16p(hipStream_t st, const vh_items &list, unsigned nitems, const vh_limb *limbs, int dir,
                             int logn, int s0, int R, int col, int first, int last, unsigned nblocks, int wide)
 {
     if (logn < 13 || logn > 16 || R < 5 || R > 8 || (!col && R != 8) || nblocks == 0) return hipErrorInvalidValue;
+    if (!list.p && nitems > VH_PASS_ITEMS) return hipErrorInvalidValue;
     if (col ? (s0 != 0 || R != logn - 8) : (s0 != logn - 8)) return hipErrorInvalidValue;
     if (!col) wide = 0;
     const unsigned G = (wide ? 512u : 256u) >> (R - 4);
@@ -1348,24 +1350,32 @@ hipError_t vh_launch_ntt16p(hipStream_t st, const vh_item *items, unsigned nitem
     const unsigned tpi = nsub / G, ntiles = tpi * nitems;
     if (wide && nblocks != UINT_MAX) nblocks = nblocks / 2 ? nblocks / 2 : 1;   // same threads per CU
     const dim3 grid(nblocks < ntiles ? nblocks : ntiles);
-#define VH_P(D, RR, CC, FF, LL, SS) VH_KL((k_ntt16p<D, RR, CC, FF, LL, SS, 256>), grid, dim3(256), 0, st, items, limbs, logn, s0, tpi, ntiles)
+    auto go = [&](const auto &args) -> hipError_t {
+        using IT = typename std::decay<decltype(args)>::type;
+#define VH_P(D, RR, CC, FF, LL, SS) \
+        VH_KL((k_ntt16p<D, RR, CC, FF, LL, SS, 256, IT>), grid, dim3(256), 0, st, list.p, args, limbs, logn, s0, tpi, ntiles)
 #define VH_PC(D, RR, FF, LL, SS) \
-    do { if (wide) VH_KL((k_ntt16p<D, RR, true, FF, LL, SS, 512>), grid, dim3(512), 0, st, items, limbs, logn, s0, tpi, ntiles); \
-         else VH_P(D, RR, true, FF, LL, SS); } while (0)
+        do { if (wide) VH_KL((k_ntt16p<D, RR, true, FF, LL, SS, 512, IT>), grid, dim3(512), 0, st, list.p, args, limbs, logn, s0, tpi, ntiles); \
+             else VH_P(D, RR, true, FF, LL, SS); } while (0)
 #define VH_P_R(D, FF, LL, SS) \
-    switch (R) { case 5: VH_PC(D, 5, FF, LL, SS); break; case 6: VH_PC(D, 6, FF, LL, SS); break; \
-                 case 7: VH_PC(D, 7, FF, LL, SS); break; default: VH_PC(D, 8, FF, LL, SS); break; }
-    // first == 2: forward first pass whose source rows are shared by items (ModUp lift)
-    if (dir == 0 && col && first == 2 && !last) { VH_P_R(0, true, false, true) }
-    else if (dir == 0 && col && first && !last) { VH_P_R(0, true, false, false) }
-    else if (dir == 0 && !col && !first && last) { VH_P(0, 8, false, false, true, false); }
-    else if (dir == 1 && !col && first && !last) { VH_P(1, 8, false, true, false, false); }
-    else if (dir == 1 && col && !first && last) { VH_P_R(1, false, true, false) }
-    else return hipErrorInvalidValue;
+        switch (R) { case 5: VH_PC(D, 5, FF, LL, SS); break; case 6: VH_PC(D, 6, FF, LL, SS); break; \
+                     case 7: VH_PC(D, 7, FF, LL, SS); break; default: VH_PC(D, 8, FF, LL, SS); break; }
+        // first == 2: forward first pass whose source rows are shared by items (ModUp lift)
+        if (dir == 0 && col && first == 2 && !last) { VH_P_R(0, true, false, true) }
+        else if (dir == 0 && col && first && !last) { VH_P_R(0, true, false, false) }
+        else if (dir == 0 && !col && !first && last) { VH_P(0, 8, false, false, true, false); }
+        else if (dir == 1 && !col && first && !last) { VH_P(1, 8, false, true, false, false); }
+        else if (dir == 1 && col && !first && last) { VH_P_R(1, false, true, false) }
+        else return hipErrorInvalidValue;
 #undef VH_P_R
 #undef VH_PC
 #undef VH_P
-    return hipGetLastError();
+        return hipGetLastError();
+    };
+    if (list.p) return go(vh_items_mem());
+    vh_items_args args;
+    for (unsigned i = 0; i < nitems; i++) args.v[i] = list.v[i];
+    return go(args);
 }
 
 // Workgroups of the pipelined pass one CU holds at once (the smallest over its instances).
