@@ -661,10 +661,11 @@ def bench_cggi(lib, args):
 
 
 def torus_flops_per_index(p) -> int:
-    """FP64 operations of one sample at one key index in k_torus_blind_rotate, counted from
-    its code (an FMA counts two; the pass-1 twiddles are formed once per kernel, outside the
-    loop).  Per transform, per 8 points (one lane): three DFT-8 (56 each), the seven slot
-    factors, pass 1's eight and pass 2's seven twiddle products (complex products of 6): 300.
+    """FP64 operations of one sample at one key index, of the algorithm with separate twiddles (an
+    FMA counts two; pass-1 twiddle powers not counted).  Per transform, per 8 points (one
+    lane): three DFT-8 (56 each), the seven slot factors, pass 1's eight and pass 2's seven twiddle
+    products (complex products of 6): 300.  (k_torus_blind_rotate's fused butterflies execute 432
+    forward and 392 inverse by this count, in 216 and 232 instructions.)
     Per key row and output component one complex multiply-add per point (8); per output
     component the partial swap's complex add and the rounding adds (2 + 2 per point)."""
     M = p.N // 2

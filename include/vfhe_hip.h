@@ -376,7 +376,7 @@ const char *vfhe_hip_device_name(void);
      "ntt.chunk_mb"      two-launch modes: MiB of rows per sub-batch, 0 = whole batch
      "ntt.tile_grid"     mode 2: passes launched one tile per workgroup instead of persistent,
                          bit 0 forward column, 1 forward row, 2 inverse row, 3 inverse column,
-                         4 the fused product's row kernel (default 15: the four passes)
+                         (default 15: the four passes; bit 4 is accepted and chooses nothing)
      "ntt.col_wide"      mode 2: 1 = column passes in 512-thread workgroups over twice the
                          columns per tile when that leaves at least two workgroups per CU
                          (default), 0 = always 256 threads
@@ -410,9 +410,9 @@ long vfhe_hip_autotune_ntt(incNTT ntt, uint64_t rows, int reps, double *us_out);
    multiply-low + add, [2] 32-bit multiply-high, [3] 32x32->64 multiply-add, [4] FP64 modular
    products (q < 2^50), [5] 64-bit Shoup modular products. */
 void vfhe_hip_probe_alu_rates(double *rates);
-/* The same for the fused product (vfhe_hip_ntt_mul_intt_batch): its row kernel one tile per
-   workgroup or persistent x its column passes at 256 / 512-by-rule / 512 threads, 6
-   candidates timed on the caller's operands (z is overwritten); the fastest is adopted and
+/* The same for the fused product (vfhe_hip_ntt_mul_intt_batch): its column passes at 256 /
+   512-by-rule / 512 threads, each as two candidates that differ in ntt.tile_grid bit 4 alone,
+   6 candidates timed on the caller's operands (z is overwritten); the fastest is adopted and
    its index returned, us_out[k] (if not null) the microseconds per call of candidate k. */
 long vfhe_hip_autotune_product(RNS_Polynomial *z, RNS_Polynomial *x, RNS_Polynomial *y, uint64_t count, int reps,
                                double *us_out);

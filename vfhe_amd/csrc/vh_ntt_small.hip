@@ -58,7 +58,7 @@ k_ntt_small(const vh_items_t<CAP> items, unsigned nitems, const vh_limb *__restr
 // transforms, the product and the inverse stay in registers.  One launch and 24 N bytes per row
 // where separate transforms and a product take 88 N bytes, three launches and temporaries.
 // 37 pairs x 3 limbs of N = 2048: 189 us a call (24 us of it kernels, the rest a temporary
-// polynomial per pair) -> 21 us.  Bound there by latency, at large batches by HBM.
+// polynomial per pair) -> 21 to 24 us.  Bound there by latency, at large batches by HBM.
 template <int LOGN, typename AR>
 __global__ void __launch_bounds__(256, 2)
 k_product_small(const vh_items items, unsigned nitems, const vh_limb *__restrict__ limbs)
@@ -260,9 +260,10 @@ k_ntt16i_row_mul(const vh_item *__restrict__ items, const vh_limb *__restrict__ 
 // Launchers
 // ---------------------------------------------------------------------------
 // Lists in the arguments (vh_items_t) by length: 16 polynomials x 4 limbs of N = 4096 took 11.1 us with the
-// list in host memory, 7.6 us so.  The argument block grows with the list it can hold because
-// the launch pays for it: a single ring product, two launches of 7 and 28 rows, takes 22.5 us with
-// 3 KiB of arguments for each and 19.5 us with these sizes (21.8 us with lists in host memory).
+// list in host memory, 7.6 us so.  The argument block grows with the list it can hold because the
+// launch pays for it: a single ring product, two launches of 7 and 28 rows whose kernels are shorter
+// than the host's part, takes 22.5 us with 3 KiB of arguments for each, 19.5 to 22.5 us with these
+// sizes and 21.2 to 22.1 us with lists in host memory.
 template <int LOGN, typename AR, unsigned CAP>
 static void vh_ntt_small_go(hipStream_t st, const vh_items_t<CAP> &items, unsigned nitems, const vh_limb *limbs, int dir)
 {
