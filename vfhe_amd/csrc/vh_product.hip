@@ -13,7 +13,7 @@
 // table instead of two, and 78 VGPRs, four workgroups per
 // CU, whose loads and butterflies overlap without an explicit prefetch.
 // Measured for 64 pairs x 24 limbs of 2^16 (2.4 GB to read and write, 0.48 ms at the rate of a large
-// copy; 0.3 ms of FP64 issue): 0.56 .. 0.68 ms, against 0.67 .. 0.83 ms for persistent workgroups
+// copy; 0.3 ms of FP64 issue): 0.56 .. 0.71 ms, against 0.67 .. 0.83 ms for persistent workgroups
 // with 16 values per thread, separate inverse tables and 234 VGPRs.
 // Grid: x = tile, y = item.
 // ---------------------------------------------------------------------------
