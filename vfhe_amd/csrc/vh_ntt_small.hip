@@ -260,10 +260,9 @@ k_ntt16i_row_mul(const vh_item *__restrict__ items, const vh_limb *__restrict__ 
 // Launchers
 // ---------------------------------------------------------------------------
 // Lists in the arguments (vh_items_t) by length: 16 polynomials x 4 limbs of N = 4096 took 11.1 us with the
-// list in host memory, 7.6 us so.  The argument block grows with the list it can hold because the
-// launch pays for it: a single ring product, two launches of 7 and 28 rows whose kernels are shorter
-// than the host's part, takes 22.5 us with 3 KiB of arguments for each, 19.5 to 22.5 us with these
-// sizes and 21.2 to 22.1 us with lists in host memory.
+// list in host memory, 7.6 us so.  The launch copies the whole block, so short lists get a short one.
+// A single ring product (launches of 7 and 28 rows) gains nothing either way: its kernels went from
+// 15 to 11 us and the host's part, 22 to 23 us with its noise of 1 us, decides.
 template <int LOGN, typename AR, unsigned CAP>
 static void vh_ntt_small_go(hipStream_t st, const vh_items_t<CAP> &items, unsigned nitems, const vh_limb *limbs, int dir)
 {
