@@ -265,7 +265,7 @@ void lwe_subto(LWE out, LWE in);                                                
 void mlwe_tensor_product(RNS_Polynomial *out, RNS_MLWE in1, RNS_MLWE in2);                            /* mlwe.c:665-709 */
 void mlwe_RNSc_GHS_hybrid_keyswitch(RNSc_MLWE out, RNSc_MLWE in, RNS_MLWE **ksk, uint64_t lvl);       /* mlwe.c:557-598 + gadget.c:22-37 */
 void mlwe_multiply(RNS_MLWE out, RNS_MLWE in1, RNS_MLWE in2, RNS_MLWE **ksk);                         /* mlwe.c:711-760 */
-void mlwe_automorphism_RNSc_GHS(RNSc_MLWE out, RNSc_MLWE in, uint64_t gen, RNS_MLWE **ksk, uint64_t lvl); /* mlwe.c:314-326 */
+void mlwe_automorphism_RNSc_GHS(RNSc_MLWE out, RNSc_MLWE in, uint64_t gen, RNS_MLWE **ksk, uint64_t lvl); /* mlwe.c:314-326; out may be in */
 RNS_MLWE_Key mlwe_new_RNS_key_from_array(uint64_t *array, uint64_t N, uint64_t r, uint64_t l, incNTT ntt, double sigma); /* mlwe.c:28-38 */
 void free_mlwe_RNS_key(RNS_MLWE_Key key);                                                             /* mlwe.c:21-26 */
 void mlwe_RNS_phase(RNS_Polynomial out, RNS_MLWE in, RNS_MLWE_Key key);                               /* mlwe.c:243-252 */

@@ -288,6 +288,22 @@ def test_automorphism(lib):
     s.check(s.pool.read_sample(out), ref, mref)
 
 
+@pytest.mark.parametrize("N,gen_exp", [(2048, 3), (8192, 1)])
+def test_automorphism_in_place(lib, N, gen_exp):
+    """mlwe_automorphism_RNSc_GHS with out == in rotates from a copy: equal to the call with its own output."""
+    s = Setup(N, 3, 1, 32 + N)
+    keys = s.outer([s.key(s.L, 1)])
+    data, cin = s.ct(1, s.lvl_mask)
+    gen = pow(5, gen_exp, 2 * N)
+    out = s.pool.sample(1, s.ext_mask)
+    lib.mlwe_automorphism_RNSc_GHS(out, cin, gen, keys, 0)
+    same = s.pool.sample(1, s.ext_mask, data)
+    s.pool.set_sample_mask(same, s.lvl_mask)
+    lib.mlwe_automorphism_RNSc_GHS(same, same, gen, keys, 0)
+    assert s.pool.sample_masks(same) == s.pool.sample_masks(out) == [s.lvl_mask] * 2
+    s.check(s.pool.read_sample(same), s.pool.read_sample(out), s.lvl_mask)
+
+
 @pytest.mark.slow
 def test_ckks_config3_shape_multiply_rescale(lib):
     """The benchmarked CKKS shape: N = 2^16, L = 24 level limbs + K = 4 special limbs, rank 1."""

@@ -2762,19 +2762,22 @@ extern "C" void mlwe_RNSc_GHS_hybrid_keyswitch(RNSc_MLWE out, RNSc_MLWE in, RNS_
 }
 
 static void automorphism_batch(const std::vector<RNS_MLWE> &outs, const std::vector<RNS_MLWE> &ins,
-                               const std::vector<uint64_t> &gens, const std::vector<RNS_MLWE **> &ksks);
+                               const std::vector<uint64_t> &gens, const std::vector<RNS_MLWE **> &ksks,
+                               bool in_place = false);
 
 extern "C" void mlwe_automorphism_RNSc_GHS(RNSc_MLWE out, RNSc_MLWE in, uint64_t gen, RNS_MLWE **ksk, uint64_t lvl)
 {
     (void)lvl;
     VH_ENTER;
-    automorphism_batch({out}, {in}, {gen}, {ksk});
+    automorphism_batch({out}, {in}, {gen}, {ksk}, true);
 }
 
 // mlwe_automorphism_RNSc_GHS (mlwe.c:314-326) for many inputs, each with its own
-// Galois element and key: permute every component, then one batched key-switch.
+// Galois element and key: permute every component into temporaries, then one batched key-switch.
+// in_place: an output may be its own input, and an input's mask components past the output's rank
+// are left out.
 static void automorphism_batch(const std::vector<RNS_MLWE> &outs, const std::vector<RNS_MLWE> &ins,
-                               const std::vector<uint64_t> &gens, const std::vector<RNS_MLWE **> &ksks)
+                               const std::vector<uint64_t> &gens, const std::vector<RNS_MLWE **> &ksks, bool in_place)
 {
     const size_t B = outs.size();
     VH_REQUIRE(B > 0 && ins.size() == B && gens.size() == B && ksks.size() == B);
@@ -2782,7 +2785,7 @@ static void automorphism_batch(const std::vector<RNS_MLWE> &outs, const std::vec
     vh_permute_rows rows;   // the temporaries' inactive rows are never read
     for (size_t bi = 0; bi < B; bi++) {
         RNS_MLWE o = outs[bi], x = ins[bi];
-        VH_REQUIRE(o != x && o->r == x->r && o->a[0]->ntt == outs[0]->a[0]->ntt);
+        VH_REQUIRE((in_place ? o->r <= x->r : o != x && o->r == x->r) && o->a[0]->ntt == outs[0]->a[0]->ntt);
         tmp[bi] = alloc_sample_raw(o->a[0]->ntt->N, o->r, o->a[0]->rns_mask, o->a[0]->ntt);
         for (uint64_t i = 0; i < o->r; i++) rows.add(tmp[bi]->a[i], x->a[i], gens[bi]);
         rows.add(tmp[bi]->b, x->b, gens[bi]);
