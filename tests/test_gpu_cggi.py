@@ -320,3 +320,37 @@ def test_fused_blind_rotation_shapes(rank, nj, count, bits):
         lib.vfhe_hip_set_option(b"br.fused", saved)
     for k in range(count):
         assert np.array_equal(got[1][k], got[0][k]), k
+
+
+@pytest.mark.parametrize("N,widths", [(1024, (50, 60, 50)), (1024, (60, 50, 60)), (1024, (60, 60, 60)), (512, (50, 60, 60)),
+                                      (8192, (60, 50, 50))])
+def test_blind_rotation_prime_widths(N, widths):
+    """Limbs of both arithmetics in one ring (FP64 below 2^50, integer above; a limb has the twiddle tables
+    of its own arithmetic only): the batch equals one mlwe_RNSc_mul_by_xai and one mgsw_CMUX per index."""
+    n, count, nj = 4, 3, len(widths) - 1
+    lib = _native.load()
+    primes = params.gen_primes(N, list(widths))
+    assert [int(q).bit_length() > 50 for q in primes] == [b > 50 for b in widths]
+    pool = rt.Pool(N, primes)
+    rng = np.random.default_rng(N + sum(widths))
+    full, level = (1 << (nj + 1)) - 1, (1 << nj) - 1
+
+    def sample(mask):
+        return pool.sample(1, mask, np.stack([rt.random_rows(rng, primes, N, mask) for _ in range(2)]))
+
+    keys = [_native.voidp_array([sample(full) for _ in range(2 * nj)]) for _ in range(n)]
+    tv = sample(level)
+    steps = rng.integers(1, 2 * N, (count, n), dtype=np.uint64)
+    rots = rng.integers(0, 2 * N, count, dtype=np.uint64)
+    acc = [pool.sample(1, level) for _ in range(count)]
+    print(f"[cggi] N={N} widths={widths}", flush=True)
+    lib.vfhe_hip_blind_rotate_tv_batch(_native.voidp_array(acc), count, tv, rots.ctypes.data_as(_native.U64P),
+                                       _native.voidp_array(keys), n, steps.ctypes.data_as(_native.U64P), nj, 1)
+    for k in range(count):
+        cur, rotated, res = (pool.sample(1, full) for _ in range(3))
+        lib.mlwe_RNSc_mul_by_xai(cur, tv, int(rots[k]))
+        for i in range(n):
+            lib.mlwe_RNSc_mul_by_xai(rotated, cur, int(steps[k, i]))
+            lib.mgsw_CMUX(res, cur, rotated, keys[i], nj, 1)
+            lib.mlwe_RNS_to_RNSc(cur, res)
+        assert np.array_equal(pool.read_sample(acc[k])[:, :nj], pool.read_sample(cur)[:, :nj]), k

@@ -3350,13 +3350,8 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
     vh_pool *P = VPOOL(t);
     const uint64_t nd = Cc * J.size(), next = E.size();
     bool fp = true;   // FP64 limbs only: the lift folds into the NTT and the inner product runs in FP64
-    bool lazy = true;
-    for (const auto *list : {&E, &J})
-        for (int e : *list) {
-            fp = fp && P->h_limbs[e].fp64;
-            lazy = lazy && ntt_kind(P->h_limbs[e]) == VH_NTT_INT;
-        }
-    const int kind = fp ? VH_NTT_FP64 : lazy ? VH_NTT_INT : VH_NTT_WIDE;
+    for (int e : E) fp = fp && P->h_limbs[e].fp64;
+    for (int j : J) fp = fp && P->h_limbs[j].fp64;
     if (fp && OPT.br_fused && N == 1024 && Cc <= 2 && divs.size() == 1 && J.size() <= VH_BR_MAXJ &&
         next == J.size() + 1) {
         // Every key index in one launch, each accumulator resident in its workgroup's LDS.
@@ -3516,8 +3511,13 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
             dj.push_back(x);
         }
     }
-    auto by_limb = [](const vh_item &a, const vh_item &b) { return a.limb < b.limb; };
-    std::stable_sort(nt.begin(), nt.end(), by_limb);    // workgroups in flight share a limb's twiddles
+    // By arithmetic (a limb has the twiddle tables of its own one only), then by limb: workgroups in
+    // flight share a limb's twiddles.
+    auto kind = [&](const vh_item &it) { return ntt_kind(P->h_limbs[it.limb]); };
+    auto by_limb = [&](const vh_item &a, const vh_item &b) {
+        return std::make_pair(kind(a), a.limb) < std::make_pair(kind(b), b.limb);
+    };
+    std::stable_sort(nt.begin(), nt.end(), by_limb);
     std::stable_sort(inv.begin(), inv.end(), by_limb);
     std::vector<uint64_t> amounts(count * n);
     for (uint64_t k = 0; k < count * n; k++) amounts[k] = steps[k] & ((N << 1) - 1);
@@ -3542,6 +3542,14 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
     auto chunks = [&](size_t total, const std::function<void(size_t, unsigned)> &f) {
         for (size_t off = 0; off < total; off += VH_MAX_GRID_Y) f(off, (unsigned)std::min<size_t>(VH_MAX_GRID_Y, total - off));
     };
+    auto transforms = [&](const std::vector<vh_item> &v, const vh_item *d_v, int dir) {
+        for (size_t a = 0, b; a < v.size(); a = b) {
+            for (b = a + 1; b < v.size() && kind(v[b]) == kind(v[a]);) b++;
+            chunks(b - a, [&](size_t off, unsigned cn) {
+                ntt_dispatch(vh_staged(d_v + a + off), cn, P->d_limbs, kind(v[a]), N, dir);
+            });
+        }
+    };
     std::vector<const uint64_t *> kptr(next * nd * Cc);
     for (uint64_t i = 0; i < n; i++) {
         VH_REQUIRE(bk[i]);
@@ -3555,7 +3563,7 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
             vh_prof_scope ps_(VH_PROF_ELTWISE);
             VH_LAUNCH(vh_launch_eltwise(S(), d_lift + off, cn, P->d_limbs, VH_OP_REDUCE, N));
         });
-        chunks(nt.size(), [&](size_t off, unsigned cn) { ntt_dispatch(vh_staged(d_nt + off), cn, P->d_limbs, kind, N, 0); });
+        transforms(nt, d_nt, 0);
         // 3. external product with bk[i]: row (ti, d, c) of the key table
         for (uint64_t d = 0; d < nd; d++) {
             const uint64_t src = d / J.size(), jj = d % J.size();
@@ -3573,7 +3581,7 @@ static void blind_rotate_core(RNS_MLWE *acc, uint64_t count, RNS_MLWE tv, const 
             VH_LAUNCH(vh_launch_keyswitch_mac(S(), d_jobs + off, cn, (unsigned)next, P->d_limbs, d_kptr, N, fp ? 1 : 0));
         });
         // 4. back to coefficient form, round-divided by the special limbs (their rows cleared)
-        chunks(inv.size(), [&](size_t off, unsigned cn) { ntt_dispatch(vh_staged(d_inv + off), cn, P->d_limbs, kind, N, 1); });
+        transforms(inv, d_inv, 1);
         if (!divs.empty()) {
             chunks(dj.size(), [&](size_t off, unsigned cn) {
                 vh_prof_scope ps_(VH_PROF_DIVISION);
