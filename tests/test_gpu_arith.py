@@ -583,6 +583,30 @@ def test_ntt_mul_intt_ragged_masks(lib, N):
         pool.free(p)
 
 
+@pytest.mark.parametrize("split", [2, 4])
+def test_split_products_bound_their_temporaries(lib, split):
+    """A batch of products on a split ring holds no more temporary memory than its y operands and one pair
+    more (what the engine parks afterwards), and every product equals the one of its pair alone."""
+    N, L, count = 65536, 11, 13
+    primes = O.gen_primes(N, [50] * L, split)
+    pool = rt.Pool(N, primes, split)
+    rng = np.random.default_rng(split)
+    x, y, z, one = ([pool.poly() for _ in range(count)] for _ in range(4))
+    for p in x + y:
+        pool.write(p, rt.random_rows(rng, primes, N))
+    arr = rt._native.voidp_array
+    lib.vfhe_hip_ntt_batch(arr(x + y), 2 * count, 0)   # operands on the device
+    lib.vfhe_hip_release_cached()
+    print(f"[split products] S={split}", flush=True)
+    lib.vfhe_hip_ntt_mul_intt_batch(arr(z), arr(x), arr(y), count)
+    assert 0 < lib.vfhe_hip_get_option(b"stat.cache_parked_bytes") <= (count + 1) * L * N * 8 + (1 << 20)
+    for k in range(count):
+        lib.vfhe_hip_ntt_mul_intt_batch(arr([one[k]]), arr([x[k]]), arr([y[k]]), 1)
+        assert np.array_equal(pool.read(z[k]), pool.read(one[k])), k
+    for p in x + y + z + one:
+        pool.free(p)
+
+
 @pytest.mark.parametrize("N", [8192, 16384, 32768, 65536])
 @pytest.mark.parametrize("tile_grid,col_wide", [(0, 0), (31, 2), (16, 0), (15, 2)])
 def test_ntt_mul_intt_grid_shapes(lib, N, tile_grid, col_wide):
