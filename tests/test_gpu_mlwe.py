@@ -7,6 +7,8 @@ correctness with real keys is covered by tests/test_gpu_ckks.py).  The pool
 layout follows modules/mlwe/python/src/vfhe/mlwe/mlwe.py:57-73: level-0 primes
 first, the special primes on top.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -286,6 +288,26 @@ def test_automorphism(lib):
     ref = np.zeros((r + 1, s.L + s.K, s.N), dtype=np.uint64)
     mref = s.octx.automorphism(ref, din, r, s.lvl_mask, gen, [keys[0][0]], s.ext_mask)
     s.check(s.pool.read_sample(out), ref, mref)
+
+
+def test_keyswitch_host_work_is_linear_in_the_batch(lib):
+    """The host time of a key-switch call per job does not grow with the batch: 2048 jobs cost at most 4
+    times as much each as 128 do (16 times if every job looked at every other)."""
+    s = Setup(256, 1, 1, 91)
+    ksk = s.outer([s.key(1, 1)])
+    ins = [s.ct(1, s.lvl_mask)[1] for _ in range(2048)]
+    outs = [s.pool.sample(1, s.ext_mask) for _ in ins]
+    per_job = {}
+    for count in (128, 2048):
+        a, b = _native.voidp_array(outs[:count]), _native.voidp_array(ins[:count])
+        for _ in range(4):
+            lib.vfhe_hip_synchronize()
+            t = time.perf_counter()
+            lib.vfhe_hip_mlwe_keyswitch_batch(a, b, count, ksk)
+            t = (time.perf_counter() - t) / count
+            per_job[count] = min(t, per_job.get(count, t))
+    print("[keyswitch] host us a job:", {k: round(v * 1e6, 2) for k, v in per_job.items()}, flush=True)
+    assert per_job[2048] <= 4 * per_job[128]
 
 
 @pytest.mark.parametrize("N,gen_exp", [(2048, 3), (8192, 1)])

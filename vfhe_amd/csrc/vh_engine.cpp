@@ -2649,12 +2649,8 @@ static void keyswitch_batch(const std::vector<RNS_MLWE> &outs, const std::vector
 
     // Back to coefficient form, then ModDown by the special primes of each job.
     std::vector<std::pair<RNS_Polynomial, RNS_Polynomial>> pairs;
-    std::map<uint64_t, std::vector<RNS_Polynomial>> by_divide;
     for (size_t bi = 0; bi < B; bi++)
-        for (auto p : comps(outs[bi])) {
-            pairs.push_back({p, p});
-            by_divide[p->rns_mask & ~ins[bi]->b->rns_mask].push_back(p);
-        }
+        for (auto p : comps(outs[bi])) pairs.push_back({p, p});
     ntt_rows(pairs, 1);
 
     // Jobs finished in one pass: at most VH_MAX_DIV special primes, one mask for every output
@@ -2668,6 +2664,7 @@ static void keyswitch_batch(const std::vector<RNS_MLWE> &outs, const std::vector
     };
     std::vector<char> fused(B, 0);
     std::map<std::tuple<uint64_t, uint64_t, uint64_t>, std::vector<size_t>> groups;   // (mask, special, rescale)
+    std::map<uint64_t, std::vector<RNS_Polynomial>> by_divide;                        // the other jobs' components
     for (size_t bi = 0; bi < B; bi++) {
         const auto oc = comps(outs[bi]);
         const uint64_t m = oc[0]->rns_mask, down = m & ~ins[bi]->b->rns_mask, keep = m & ~down;
@@ -2678,17 +2675,9 @@ static void keyswitch_batch(const std::vector<RNS_MLWE> &outs, const std::vector
             ok = oc[c]->rns_mask == m && (!pass[bi][c] || (pass[bi][c]->rns_mask & keep) == keep);
         fused[bi] = ok;
         if (ok) groups[std::make_tuple(m, down, resc)].push_back(bi);
+        else for (auto p : oc) by_divide[p->rns_mask & ~ins[bi]->b->rns_mask].push_back(p);
     }
-    for (auto &g : by_divide) {
-        std::vector<RNS_Polynomial> rest;
-        for (auto p : g.second) {
-            bool f = false;
-            for (size_t bi = 0; bi < B && !f; bi++)
-                if (fused[bi]) for (auto o : comps(outs[bi])) f = f || o == p;
-            if (!f) rest.push_back(p);
-        }
-        if (g.first) run_division(rest, g.first, true);
-    }
+    for (auto &g : by_divide) if (g.first) run_division(g.second, g.first, true);
     std::vector<vh_item> adds;
     for (size_t bi = 0; bi < B; bi++) {
         if (fused[bi]) continue;
