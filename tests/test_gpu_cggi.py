@@ -282,7 +282,7 @@ def test_bootstrap_batch_shape_n630_N1024():
 
 @pytest.mark.parametrize("rank,nj,count,bits", [
     (1, 2, 1, 50), (1, 2, 259, 50), (1, 1, 3, 50), (1, 1, 257, 50), (1, 3, 5, 50), (1, 3, 258, 50),
-    (0, 1, 2, 50), (0, 2, 3, 50), (0, 2, 257, 50), (0, 3, 2, 50), (1, 2, 4, 30),
+    (0, 1, 2, 50), (0, 1, 515, 50), (0, 2, 3, 50), (0, 2, 257, 50), (0, 3, 2, 50), (1, 2, 4, 30),
 ])
 def test_fused_blind_rotation_shapes(rank, nj, count, bits):
     """Every form of the one-launch blind rotation (one accumulator per workgroup with one or two

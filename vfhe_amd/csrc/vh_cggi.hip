@@ -43,11 +43,19 @@
 namespace {
 constexpr int BN = 1024, BH = 512, BSCR = 576;   // ring, half, doubles of a wave's exchange slice
 
+// One component and one level limb: the t row lies over the digits, and the halves go through the waves'
+// slices as every last component's do.  70 KiB a workgroup instead of 116, two of them on a CU: 513
+// accumulators at n = 60 take 0.69 ms (0.87), 1024 take 0.70 ms (0.89).  At more level limbs still one
+// workgroup would fit, and the tighter layout is slower (two limbs, 1 accumulator: 0.58 ms against 0.54).
+template <int C, int NJ> constexpr bool br_lean() { return C == 1 && NJ == 1; }
 template <int C, int NJ> constexpr int br_reg()   // doubles: the rows, or the exchanged halves and one t row
 {
-    return (C * NJ > NJ + 2 ? C * NJ : NJ + 2) * BN;
+    return (br_lean<C, NJ>() || C * NJ > NJ + 2 ? C * NJ : NJ + 2) * BN;
 }
-template <int C, int NJ, int G> constexpr int br_per_acc() { return br_reg<C, NJ>() + 2 * G * (NJ + 1) * BSCR + BN; }
+template <int C, int NJ, int G> constexpr int br_per_acc()
+{
+    return br_reg<C, NJ>() + 2 * G * (NJ + 1) * BSCR + (br_lean<C, NJ>() ? 0 : BN);
+}
 template <int C, int NJ, int NA, int G> constexpr int br_lds() { return NA * br_per_acc<C, NJ, G>() + (NJ + 1) * BN; }
 }  // namespace
 
@@ -70,7 +78,7 @@ k_blind_rotate(const vh_br_params P, const vh_limb *__restrict__ limbs, uint64_t
     const bool live = k < count;   // a slot past the end works on zeros and stores nothing
     double *reg = lds + ac * PER;
     double *scr = reg + REG + ((g * next + w) * 2 + h) * BSCR, *pscr = reg + REG + ((g * next + w) * 2 + 1 - h) * BSCR;
-    double *tlast = reg + REG + 2 * G * next * BSCR, *tfirst = reg + next * BN;
+    double *tlast = br_lean<C, NJ>() ? reg : reg + REG + 2 * G * next * BSCR, *tfirst = reg + next * BN;
     const double *tw = lds + NA * PER + w * BN;
     for (int e = threadIdx.x; e < next * BN; e += blockDim.x)
         lds[NA * PER + e] =
@@ -354,7 +362,7 @@ hipError_t vh_launch_blind_rotate(hipStream_t st, const vh_br_params &P, const v
     if (P.C < 1 || P.C > 2 || P.nJ < 1 || P.nJ > VH_BR_MAXJ || P.next != P.nJ + 1 || P.next > VH_BR_MAXE ||
         P.sp < 0 || P.sp >= P.next || count == 0 || (tvp && !rot))
         return hipErrorInvalidValue;
-    // One workgroup fits a CU.  Up to one accumulator per CU, each takes twice the waves (G = 2):
+    // One workgroup fits a CU (two at one component and one level limb).  Up to one accumulator per CU, each takes twice the waves (G = 2):
     // 8 accumulators of n = 630 take 9.0 ms (12.3 ms with G = 1).  Beyond, two accumulators
     // share a workgroup: 300 take 18.5 ms where one per CU would take two rounds of 9.
     const int na = count > cus && P.nJ < 3 ? 2 : 1, g = na == 1 && P.C == 2 && P.nJ < 3 ? 2 : 1;
