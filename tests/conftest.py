@@ -20,6 +20,12 @@ def lib():
 
 
 @pytest.fixture(scope="session")
+def cus(lib):
+    """Compute units of the device (the engine's placement probe ran four workgroups for each)."""
+    return sum(lib.vfhe_hip_get_option(b"probe.xcd%d" % k) for k in range(8)) // 4
+
+
+@pytest.fixture(scope="session")
 def oracle():
     from oracle import oracle as O
     return O

@@ -90,6 +90,30 @@ def test_small_ntt_batch_register_kernel(lib, N):
         lib.vfhe_hip_set_option(b"ntt.small", saved)
 
 
+@pytest.mark.parametrize("per_cu_x2,small", [(0, False), (2, False), (3, False), (4, True)])
+def test_integer_transforms_of_512_points(lib, cus, per_cu_x2, small):
+    """Integer limbs at N = 512: few rows go to the radix-2 kernel (quicker there), more than 3 for 2 CUs to
+    the register kernel, both directions against the oracle."""
+    N, rows = 512, max(1, per_cu_x2 * cus // 2)
+    primes = [int(O.lib().o_next_special_prime(1 << 60, N, 1))]
+    pool, c, rng = rt.Pool(N, primes), O.Ctx(N, primes), np.random.default_rng(rows)
+    xs = [rt.random_rows(rng, primes, N) for _ in range(rows)]
+    ps = [pool.poly(x) for x in xs]
+    arr = rt._native.voidp_array(ps)
+    print(f"[512-point integer] rows={rows}", flush=True)
+    n0 = lib.vfhe_hip_get_option(b"stat.ntt_small_launches")
+    lib.vfhe_hip_ntt_batch(arr, rows, 0)
+    for x, p in zip(xs, ps):
+        ref = x.copy()
+        c.to_ntt(ref, ref, 1)
+        assert np.array_equal(pool.read(p), ref)
+    lib.vfhe_hip_ntt_batch(arr, rows, 1)
+    assert all(np.array_equal(pool.read(p), x) for p, x in zip(ps, xs))
+    assert lib.vfhe_hip_get_option(b"stat.ntt_small_launches") - n0 == (2 if small else 0)
+    for p in ps:
+        pool.free(p)
+
+
 def test_block_cache_cap_and_release(lib):
     """The device block cache keeps at most cache.max_mb parked, evicting the least recently parked
     blocks (results unchanged), and vfhe_hip_release_cached empties it."""

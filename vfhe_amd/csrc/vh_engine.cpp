@@ -782,7 +782,15 @@ static int col_wide(unsigned items, int logn)
 enum { VH_NTT_WIDE = 0, VH_NTT_FP64 = 1, VH_NTT_INT = 2 };
 static int ntt_kind(const vh_limb &h) { return h.fp64 ? VH_NTT_FP64 : h.q < (1ULL << 62) ? VH_NTT_INT : VH_NTT_WIDE; }
 
-static bool ntt_is_small(int kind, uint64_t n) { return kind != VH_NTT_WIDE && n >= 512 && n <= 4096 && OPT.ntt_small; }
+// Whole transforms in registers.  Not integer ones of 512 points until 3 rows for 2 CUs: a thread's chain
+// of 16 values costs more there than the radix-2 kernel's stages of one butterfly each (1 row 8.0 us
+// against 7.3 forward, 8.9 against 7.0 inverse; 256 rows 9.6 against 8.3, 10.0 against 8.1; 384 rows
+// alike, 1536 rows 28 against 32).
+static bool ntt_is_small(int kind, uint64_t n, unsigned cnt)
+{
+    return kind != VH_NTT_WIDE && n >= 512 && n <= 4096 && OPT.ntt_small &&
+           !(kind == VH_NTT_INT && n == 512 && cnt <= (unsigned)C.cus * 3 / 2);
+}
 static void ntt_small_launch(const vh_items &items, unsigned cnt, const vh_limb *d_limbs, int kind, uint64_t n, int dir)
 {
     // whole transforms in registers, 4096/N of them per workgroup
@@ -794,11 +802,11 @@ static void ntt_small_launch(const vh_items &items, unsigned cnt, const vh_limb 
 
 static vh_items vh_staged(const vh_item *d) { vh_items w; w.p = d; return w; }
 
-// The longest list ntt_dispatch takes in kernel arguments (0: every list must be staged).
-static unsigned ntt_inline_cap(int kind, uint64_t n)
+// The longest list ntt_dispatch takes in kernel arguments for cnt items (0: the list must be staged).
+static unsigned ntt_inline_cap(int kind, uint64_t n, unsigned cnt)
 {
     return n >= 8192 && n <= 65536 && kind == VH_NTT_FP64 && OPT.ntt_mode == 2 && C.pipe_blocks > 0 &&
-           OPT.ntt_chunk_mb <= 0 ? VH_PASS_ITEMS : ntt_is_small(kind, n) ? VH_INLINE_ITEMS : 0;
+           OPT.ntt_chunk_mb <= 0 ? VH_PASS_ITEMS : ntt_is_small(kind, n, cnt) ? VH_INLINE_ITEMS : 0;
 }
 
 // Launches the transforms of `cnt` work items (device list d_items, all of one
@@ -807,7 +815,7 @@ static void ntt_dispatch(const vh_items &list, unsigned cnt, const vh_limb *d_li
 {
     const int logn = ilog2(n), fp = kind == VH_NTT_FP64;
     const vh_item *d_items = list.p;   // null: the list is in `list`, at most ntt_inline_cap items
-    VH_REQUIRE(d_items || cnt <= ntt_inline_cap(kind, n));
+    VH_REQUIRE(d_items || cnt <= ntt_inline_cap(kind, n, cnt));
     if (fp && logn >= 13 && logn <= 16 && OPT.ntt_mode == 1 && C.xcd_ok) {
         // Persistent kernel: both passes of every transform on one XCD, the
         // intermediate exchanged through that XCD's L2.
@@ -850,7 +858,7 @@ static void ntt_dispatch(const vh_items &list, unsigned cnt, const vh_limb *d_li
                 { vh_prof_scope ps_(VH_PROF_NTT_FP64); VH_LAUNCH(vh_launch_ntt16(S(), ci, cc, d_limbs, 1, logn, 0, R1, 1, 0, 1)); }
             }
         }
-    } else if (ntt_is_small(kind, n)) {
+    } else if (ntt_is_small(kind, n, cnt)) {
         ntt_small_launch(list, cnt, d_limbs, kind, n, dir);
     } else if (kind == VH_NTT_INT && logn >= 13 && logn <= 16) {
         // two register passes, column then row (inverse: row then column)
@@ -888,7 +896,7 @@ static void run_ntt(std::vector<vh_item> &items, const vh_limb *d_limbs, const v
         for (size_t off = 0; off < v.size(); off += VH_MAX_GRID_Y) {
             const unsigned cnt = (unsigned)std::min<size_t>(VH_MAX_GRID_Y, v.size() - off);
             std::vector<vh_item> chunk(v.begin() + off, v.begin() + off + cnt);
-            ntt_dispatch(vh_work(chunk, ntt_inline_cap(kind, n)), cnt, d_limbs, kind, n, dir);
+            ntt_dispatch(vh_work(chunk, ntt_inline_cap(kind, n, cnt)), cnt, d_limbs, kind, n, dir);
         }
     }
 }
