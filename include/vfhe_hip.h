@@ -375,8 +375,8 @@ const char *vfhe_hip_device_name(void);
                          0: two launches of the plain pass kernel; 1: persistent per-XCD kernel
      "ntt.chunk_mb"      two-launch modes: MiB of rows per sub-batch, 0 = whole batch
      "ntt.tile_grid"     mode 2: passes launched one tile per workgroup instead of persistent,
-                         bit 0 forward column, 1 forward row, 2 inverse row, 3 inverse column,
-                         (default 15: the four passes; bit 4 is accepted and chooses nothing)
+                         bit 0 forward column, 1 forward row, 2 inverse row, 3 inverse column
+                         (default 15: the four passes; bit 4 is accepted and dropped)
      "ntt.col_wide"      mode 2: 1 = column passes in 512-thread workgroups over twice the
                          columns per tile when that leaves at least two workgroups per CU
                          (default), 0 = always 256 threads
@@ -411,9 +411,10 @@ long vfhe_hip_autotune_ntt(incNTT ntt, uint64_t rows, int reps, double *us_out);
    products (q < 2^50), [5] 64-bit Shoup modular products. */
 void vfhe_hip_probe_alu_rates(double *rates);
 /* The same for the fused product (vfhe_hip_ntt_mul_intt_batch): its column passes at 256 /
-   512-by-rule / 512 threads, each as two candidates that differ in ntt.tile_grid bit 4 alone,
-   6 candidates timed on the caller's operands (z is overwritten); the fastest is adopted and
-   its index returned, us_out[k] (if not null) the microseconds per call of candidate k. */
+   512-by-rule / 512 threads (ntt.col_wide 0 / 1 / 2) timed on the caller's operands (z is
+   overwritten), the fastest adopted.  Each setting c counts as two candidates, 2 c and 2 c + 1:
+   both entries of us_out (6, if not null) hold its microseconds per call, and the odd index of
+   the fastest is returned. */
 long vfhe_hip_autotune_product(RNS_Polynomial *z, RNS_Polynomial *x, RNS_Polynomial *y, uint64_t count, int reps,
                                double *us_out);
 /* The same for the CKKS multiply batch (vfhe_hip_mlwe_multiply_batch): column-pass width x

@@ -714,8 +714,8 @@ def test_mul_modq_against_bigint(lib):
 
 
 def test_product_autotuner_adopts_a_timed_schedule(lib):
-    """vfhe_hip_autotune_product times its 6 schedules, adopts the fastest (bit 4 of ntt.tile_grid
-    and ntt.col_wide), and the fused product afterwards equals the oracle."""
+    """vfhe_hip_autotune_product times its three schedules (two candidate indexes each), adopts the fastest
+    (ntt.col_wide; ntt.tile_grid stays), and the fused product afterwards equals the oracle."""
     N, L, P = 16384, 3, 4
     primes = O.gen_primes(N, [50] * L)
     pool = rt.Pool(N, primes)
@@ -748,6 +748,33 @@ def test_product_autotuner_adopts_a_timed_schedule(lib):
     finally:
         for k, v in before.items():
             lib.vfhe_hip_set_option(k, v)
+
+
+def test_dropped_tile_grid_bit(lib):
+    """ntt.tile_grid bit 4 chooses nothing: it is dropped where the option is set (so that graph plans do not
+    differ by it), and the product tuner gives both indexes of a pair the one time it measured."""
+    N, count = 8192, 2
+    pool = rt.Pool(N, O.gen_primes(N, [50]))
+    x, y, z = ([pool.poly() for _ in range(count)] for _ in range(3))
+    keys = (b"ntt.tile_grid", b"ntt.col_wide")
+    before = {k: lib.vfhe_hip_get_option(k) for k in keys}
+    us = (ctypes.c_double * 6)()
+    arr = rt._native.voidp_array
+    try:
+        for value, kept in ((31, 15), (16, 0), (15, 15)):
+            assert lib.vfhe_hip_set_option(b"ntt.tile_grid", value) == 0
+            assert lib.vfhe_hip_get_option(b"ntt.tile_grid") == kept
+        print("[autotune product] pairs", flush=True)
+        best = lib.vfhe_hip_autotune_product(arr(z), arr(x), arr(y), count, 2, us)
+        assert best in (1, 3, 5) and all(u > 0 for u in us)
+        assert all(us[2 * c] == us[2 * c + 1] for c in range(3)) and us[best] == min(us)
+        assert lib.vfhe_hip_get_option(b"ntt.tile_grid") == 15
+        lib.vfhe_hip_autotune_product(arr(z), arr(x), arr(y), count, 1, None)
+    finally:
+        for k, v in before.items():
+            lib.vfhe_hip_set_option(k, v)
+    for p in x + y + z:
+        pool.free(p)
 
 
 def test_alu_rate_probe(lib):

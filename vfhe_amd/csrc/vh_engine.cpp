@@ -184,7 +184,7 @@ struct vh_opts {
     long ntt_col_wide = 1;    // pipelined column passes: 512-thread workgroups over 32-column tiles
     long ntt_tile_grid = 15;   // pipelined passes launched one tile per workgroup instead of
                               // persistent: bit 0 forward column, 1 forward row, 2 inverse row,
-                              // 3 inverse column (bit 4 chooses nothing)
+                              // 3 inverse column (bit 4 is dropped where the option is set)
     long xcd_lag = 3;         // persistent mode: queue slots between an item's two passes
     long xcd_occ = 2;         // persistent mode: workgroups per CU (2 or 4)
     long xcd_l2 = 1;          // persistent mode: the first pass stores its intermediate with
@@ -224,7 +224,7 @@ static void vh_ensure()
     C.pipe_blocks = (unsigned)(C.cus * vh_ntt16p_occupancy());
     if (const char *e = getenv("VFHE_HIP_NTT_MODE")) OPT.ntt_mode = atol(e);
     if (const char *e = getenv("VFHE_HIP_NTT_CHUNK_MB")) OPT.ntt_chunk_mb = atol(e);
-    if (const char *e = getenv("VFHE_HIP_NTT_TILE_GRID")) OPT.ntt_tile_grid = atol(e);
+    if (const char *e = getenv("VFHE_HIP_NTT_TILE_GRID")) OPT.ntt_tile_grid = atol(e) & ~16L;
     if (const char *e = getenv("VFHE_HIP_NTT_COL_WIDE")) OPT.ntt_col_wide = atol(e);
     if (const char *e = getenv("VFHE_HIP_XCD_LAG")) OPT.xcd_lag = atol(e);
     if (const char *e = getenv("VFHE_HIP_XCD_OCC")) OPT.xcd_occ = atol(e);
@@ -1257,7 +1257,7 @@ extern "C" int vfhe_hip_set_option(const char *key, long value)
     if (!key) return -1;
     if (!strcmp(key, "ntt.mode")) OPT.ntt_mode = value;
     else if (!strcmp(key, "ntt.chunk_mb")) OPT.ntt_chunk_mb = value;
-    else if (!strcmp(key, "ntt.tile_grid")) OPT.ntt_tile_grid = value;
+    else if (!strcmp(key, "ntt.tile_grid")) OPT.ntt_tile_grid = value & ~16L;
     else if (!strcmp(key, "ntt.col_wide")) OPT.ntt_col_wide = value;
     else if (!strcmp(key, "ntt.xcd_lag")) OPT.xcd_lag = value < 0 ? 0 : value;
     else if (!strcmp(key, "ntt.xcd_occupancy")) OPT.xcd_occ = value;
@@ -4543,9 +4543,8 @@ extern "C" long vfhe_hip_autotune_ntt(incNTT ntt, uint64_t rows, int reps, doubl
     }
     VH_CHECK(hipEventDestroy(e0));
     VH_CHECK(hipEventDestroy(e1));
-    // Adopt the winner's timed settings only: the fused product's row-kernel bit (tile_grid
-    // bit 4) keeps its value, and the 512-thread column rule is enabled only when the winning
-    // candidate's timed launches actually ran wide (otherwise the caller's setting stays).
+    // Adopt the winner's timed settings only: the 512-thread column rule is enabled only when the
+    // winning candidate's timed launches actually ran wide (otherwise the caller's setting stays).
     OPT = saved;
     OPT.ntt_mode = VH_SCHEDS[best].mode; OPT.ntt_chunk_mb = VH_SCHEDS[best].chunk_mb;
     OPT.xcd_lag = VH_SCHEDS[best].lag; OPT.xcd_occ = VH_SCHEDS[best].occ;
@@ -4596,20 +4595,19 @@ static long autotune_generic(long nc, const std::function<void(long)> &apply, co
 }
 
 // The fused product's schedule: its column passes at 256 threads, 512 threads by the occupancy rule,
-// or 512 threads always (ntt.col_wide 0 / 1 / 2), each timed twice on the caller's operands (z is
-// overwritten): 6 candidates, of which those that differ in ntt.tile_grid bit 4 alone run alike.
+// or 512 threads always (ntt.col_wide 0 / 1 / 2), timed on the caller's operands (z is overwritten).
+// The interface counts 6 candidates, 2 k and 2 k + 1 for ntt.col_wide = k, once told apart by the row
+// kernel's form: us_out gives both the same time, and the odd one is returned.
 extern "C" long vfhe_hip_autotune_product(RNS_Polynomial *z, RNS_Polynomial *x, RNS_Polynomial *y, uint64_t count,
                                           int reps, double *us_out)
 {
     VH_ENTER;
     VH_REQUIRE(z && x && y && count > 0);
-    return autotune_generic(
-        6,
-        [&](long k) {
-            OPT.ntt_tile_grid = (OPT.ntt_tile_grid & ~16L) | ((k & 1) ? 0L : 16L);
-            OPT.ntt_col_wide = k >> 1;
-        },
-        [&] { ntt_mul_intt(z, x, y, count); }, reps, us_out);
+    double us[3];
+    const long best = autotune_generic(
+        3, [&](long k) { OPT.ntt_col_wide = k; }, [&] { ntt_mul_intt(z, x, y, count); }, reps, us);
+    for (int k = 0; k < 6 && us_out; k++) us_out[k] = us[k >> 1];
+    return 2 * best + 1;
 }
 
 // The CKKS multiply batch's schedule: column passes (the ModUp pass and the inverse ones)
