@@ -56,9 +56,13 @@ k_ntt_small(const vh_items_t<CAP> items, unsigned nitems, const vh_limb *__restr
 
 // z = INTT(NTT(x) NTT(y)) of whole rows: x in it.src, y in it.src2, z in it.dst; both forward
 // transforms, the product and the inverse stay in registers.  One launch and 24 N bytes per row
-// where separate transforms and a product take 88 N bytes, three launches and temporaries.
+// where separate transforms and a product take 72 N bytes, three launches and temporaries.
 // 37 pairs x 3 limbs of N = 2048: 189 us a call (24 us of it kernels, the rest a temporary
-// polynomial per pair) -> 21 to 24 us.  Bound there by latency, at large batches by HBM.
+// polynomial per pair) -> 21 to 24 us.  Bound by latency at every batch: 64 pairs x 24 limbs of
+// N = 4096 take 112 us for 151 MB (1.3 TB/s) and 35 us of VALU issue, two waves a SIMD (210 to 248
+// VGPRs from N = 1024) waiting for 72% of their time.  The integer instances want more registers
+// than that leaves and spill 48 at N = 2048 (188 bytes a lane), 82 at 4096 (324 bytes): one pair of
+// 60 bits at N = 4096 takes 35 us, and took 81 in separate launches of the radix-2 kernel.
 template <int LOGN, typename AR>
 __global__ void __launch_bounds__(256, 2)
 k_product_small(const vh_items items, unsigned nitems, const vh_limb *__restrict__ limbs)
@@ -259,10 +263,12 @@ k_ntt16i_row_mul(const vh_item *__restrict__ items, const vh_limb *__restrict__ 
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-// Lists in the arguments (vh_items_t) by length: 16 polynomials x 4 limbs of N = 4096 took 11.1 us with the
-// list in host memory, 7.6 us so.  The launch copies the whole block, so short lists get a short one.
+// Lists in the arguments (vh_items_t): 16 polynomials x 4 limbs of N = 4096 took 11.1 us with the list in
+// host memory, 7.6 us so.  The launch copies the whole block, so lists of at most 16 rows (and staged
+// ones) get a short one.  That is worth little: 0.1 us of 5.5 to 7 at best on a short list, 0.2 of 19 on
+// staged lists of 512 rows.  A third block of 32 rows changed nothing (17 to 32 rows alike to 0.1 us).
 // A single ring product (launches of 7 and 28 rows) gains nothing either way: its kernels went from
-// 15 to 11 us and the host's part, 22 to 23 us with its noise of 1 us, decides.
+// 15 to 11 us and the host's part, 17 to 23 us from run to run, decides.
 template <int LOGN, typename AR, unsigned CAP>
 static void vh_ntt_small_go(hipStream_t st, const vh_items_t<CAP> &items, unsigned nitems, const vh_limb *limbs, int dir)
 {
@@ -277,7 +283,6 @@ hipError_t vh_launch_ntt_small(hipStream_t st, const vh_items &items, unsigned n
     if (logn < 9 || logn > 12 || nitems == 0) return hipErrorInvalidValue;
 #define VH_SMALL(LG, AR)                                                                                    \
         if (items.p || nitems <= 16) vh_ntt_small_go<LG, AR>(st, vh_items_cut<16>(items, nitems), nitems, limbs, dir); \
-        else if (nitems <= 32) vh_ntt_small_go<LG, AR>(st, vh_items_cut<32>(items, nitems), nitems, limbs, dir);       \
         else vh_ntt_small_go<LG, AR>(st, items, nitems, limbs, dir);
 #define VH_SIZE(LG) case LG: if (fp) { VH_SMALL(LG, vh_ar_fp) } else { VH_SMALL(LG, vh_ar_int) } break;
     switch (logn) { VH_SIZE(9) VH_SIZE(10) VH_SIZE(11) VH_SIZE(12) }
