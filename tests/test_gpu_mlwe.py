@@ -242,7 +242,7 @@ def test_moddown_without_rescale_fp64_against_integer(lib, N, L, K, batch):
 @pytest.mark.parametrize("rescale", [False, True])
 def test_multiply_pass_through_folded_into_key_mac(lib, rescale):
     """ks.fold = 1: the tensor's linear and constant slots stay in NTT form and enter the fused
-    key inner product as P * d (k_ntt16_row_mac), instead of being added after the ModDown.
+    key inner product as P * d (k_row_mac), instead of being added after the ModDown.
     Bit-equal to ks.fold = 0 and to the oracle (mlwe.c:711-760, then ckks.py:128-148)."""
     s = Setup(8192, 4, 2, 77 + rescale)
     r, m = 1, s.lvl_mask

@@ -3882,8 +3882,9 @@ extern "C" int vfhe_hip_ntt_batch_noalloc(RNS_Polynomial *polys, uint64_t count,
         const uint64_t m = polys[i]->rns_mask & (t->l >= 64 ? ~0ULL : ((1ULL << t->l) - 1));
         rows += (uint64_t)__builtin_popcountll(m) * t->split_degree;
     }
-    // per row: a 48-byte work item and two 4-byte counters; per launch group (at most
-    // two: FP64 and integer limbs) the 256-byte roundings and the 16 queue tickets
+    // per row: a 48-byte work item and two 4-byte counters; per launch group (at most three, one
+    // for each arithmetic) the 256-byte rounding of its list, and for the FP64 one that of its
+    // counters and the 16 queue tickets: under 1.2 KiB
     const size_t need = rows * (sizeof(vh_item) + 8) + 2048;
     if (need > VH_SCRATCH_BYTES) {
         fprintf(stderr, "vfhe hip engine: vfhe_hip_ntt_batch_noalloc: %lu limb rows need %zu bytes of scratch, "
