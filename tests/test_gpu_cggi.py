@@ -13,6 +13,7 @@ benchmark's bootstrap shape: LWE dimension 630, N = 1024, 1024 ciphertexts of
 """
 import ctypes
 import random
+import time
 
 import numpy as np
 import pytest
@@ -354,3 +355,70 @@ def test_blind_rotation_prime_widths(N, widths):
             lib.mgsw_CMUX(res, cur, rotated, keys[i], nj, 1)
             lib.mlwe_RNS_to_RNSc(cur, res)
         assert np.array_equal(pool.read_sample(acc[k])[:, :nj], pool.read_sample(cur)[:, :nj]), k
+
+
+@pytest.mark.parametrize("rank,nj,count", [(1, 2, 1), (1, 2, 9), (1, 2, 259), (1, 1, 258), (1, 3, 4), (0, 1, 515)])
+def test_fused_blind_rotation_skips_zero_exponents(rank, nj, count):
+    """Exponents of 0 (the reference's skipped index) for some accumulators at an index, for all of them (left out
+    of the kernel's tables; the first, successive and last indexes) and for whole accumulators, against the
+    launch sequence per index."""
+    N, n = 1024, 6
+    lib = _native.load()
+    primes = params.gen_primes(N, [50] * (nj + 1))
+    pool = rt.Pool(N, primes)
+    rng = np.random.default_rng(8000 + 100 * nj + 10 * rank + count)
+    full, level = (1 << (nj + 1)) - 1, (1 << nj) - 1
+
+    def sample(mask):
+        return pool.sample(rank, mask, np.stack([rt.random_rows(rng, primes, N, mask) for _ in range(rank + 1)]))
+
+    keys = [_native.voidp_array([sample(full) for _ in range((rank + 1) * nj)]) for _ in range(n)]
+    tv = sample(level)
+    steps = rng.integers(1, 2 * N, (count, n), dtype=np.uint64) * rng.integers(0, 2, (count, n), dtype=np.uint64)
+    steps[:, [0, 1, n - 1]] = 0
+    for k in range(0, count, 5):   # whole accumulators, some with their neighbour
+        steps[k:k + 1 + k % 2] = 0 if k else steps[k:k + 1]
+    steps[-1, 2] = 3
+    rots = rng.integers(0, 2 * N, count, dtype=np.uint64)
+    saved = lib.vfhe_hip_get_option(b"br.fused")
+    got = {}
+    try:
+        for fused in (1, 0):
+            assert lib.vfhe_hip_set_option(b"br.fused", fused) == 0
+            acc = [pool.sample(rank, level) for _ in range(count)]
+            print(f"[cggi] zero exponents: rank={rank} limbs={nj} count={count} fused={fused}", flush=True)
+            lib.vfhe_hip_blind_rotate_tv_batch(_native.voidp_array(acc), count, tv, rots.ctypes.data_as(_native.U64P),
+                                               _native.voidp_array(keys), n, steps.ctypes.data_as(_native.U64P), nj, 1)
+            got[fused] = [pool.read_sample(c)[:, :nj] for c in acc]
+    finally:
+        lib.vfhe_hip_set_option(b"br.fused", saved)
+    for k in range(count):
+        assert np.array_equal(got[1][k], got[0][k]), k
+
+
+def test_trivial_samples_cost_no_rotation():
+    """A batch whose exponents are all 0 (trivial samples) has nothing to rotate by: it takes under a tenth of the
+    time of nonzero exponents, and leaves X^rot tv."""
+    N, n, count = 1024, 630, 8
+    lib = _native.load()
+    primes = params.gen_primes(N, [50] * 3)
+    pool = rt.Pool(N, primes)
+    rng = np.random.default_rng(9)
+    row = [pool.sample(1, 7, np.stack([rt.random_rows(rng, primes, N) for _ in range(2)])) for _ in range(4)]
+    keys, tv = _native.voidp_array([_native.voidp_array(row)] * n), pool.sample(1, 3)
+    rots = np.zeros(count, dtype=np.uint64)
+    took = {}
+    for name, steps in (("nonzero", rng.integers(1, 2 * N, (count, n), dtype=np.uint64)),
+                        ("zero", np.zeros((count, n), dtype=np.uint64))):
+        acc = [pool.sample(1, 3) for _ in range(count)]
+        for _ in range(3):
+            lib.vfhe_hip_synchronize()
+            t = time.perf_counter()
+            lib.vfhe_hip_blind_rotate_tv_batch(_native.voidp_array(acc), count, tv, rots.ctypes.data_as(_native.U64P),
+                                               keys, n, steps.ctypes.data_as(_native.U64P), 2, 1)
+            lib.vfhe_hip_synchronize()
+            took[name] = min(time.perf_counter() - t, took.get(name, 1.0))
+    print("[cggi] ms:", {k: round(v * 1e3, 2) for k, v in took.items()}, flush=True)
+    assert took["zero"] < took["nonzero"] / 10
+    for c in acc:   # rot = 0
+        assert np.array_equal(pool.read_sample(c)[:, :2], pool.read_sample(tv)[:, :2])
