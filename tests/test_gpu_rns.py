@@ -162,7 +162,7 @@ def test_base_conversion_and_scaled_lift(lib, N, L, split):
     active_eq(pool.read(out2), ref, out_mask)
 
 
-@pytest.mark.parametrize("N,L,split", CASES + [(65536, 4, 1)])
+@pytest.mark.parametrize("N,L,split", CASES + [(65536, 4, 1), (65536, 9, 1), (65536, 10, 4)])   # 2^19 elements and more
 def test_permute(lib, N, L, split):
     primes, pool, octx, rng = setup(N, L, split, 6)
     m = pool.full_mask() & ~0b10
